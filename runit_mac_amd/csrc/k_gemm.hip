@@ -794,7 +794,15 @@ struct PrepSum {
     const float* res;
     float* y;
     uint32_t splits, crow;
+    uint32_t full, nch;  // wide GEMM: its first `full` tiles are unsplit (wide_splits)
 };
+
+// K splits of the 256-column tile that holds column n of chunk ch in the
+// partial sums of a wide GEMM (k_gemmw.hip): tiles in the order [column tile]
+// [chunk], the first `full` of them unsplit.
+RT_DEV uint32_t wide_splits(uint32_t full, uint32_t splits, uint32_t n, uint32_t tile, uint32_t nch, uint32_t ch) {
+    return n / tile * nch + ch < full ? 1 : splits;
+}
 
 // The row of a preparation given as the split partials of the multi-query
 // attention (k_attn_mq_f32_hd*, parts-only, one sequence): element (head h,
@@ -805,6 +813,43 @@ struct PrepAttn {
     const float* ml;
     uint32_t nsp, G, hd, cgs;
 };
+
+// One float4 of the operands of k_gemmw.hip (chunks of 64 rows): [chunk]
+// [stage of 2 records][record][MFMA p][32-row tile][hi, lo][64 lanes] entries
+// of 8 halves; lane 32·h + row holds elements 16p + 8h .. + 7 of the record in
+// the order 0 2 1 3 4 6 5 7.  A record past K is zero.  stab: the record sums
+// of each super-block as f16 pairs hi + lo of Σx·2^-6, [chunk][super-block]
+// [tile][32·(hi, lo) + row][8 records in the same order].
+RT_DEV void prep_store_wide(uint2* __restrict__ aops, float* __restrict__ stab, uint32_t m,
+                            uint32_t rec, uint32_t qf, uint32_t nrec, const _Float16 (&h)[4],
+                            const _Float16 (&l)[4]) {
+    auto two = [](_Float16 a, _Float16 b) {
+        return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
+    };
+    const uint32_t ch = m / 64, t = m / 32 % 2, mm = m % 32;
+    const uint32_t p = qf >> 2, hh = (qf >> 1) & 1;
+    uint2* base = aops + ((((size_t)ch * ((nrec + 1) / 2) * 2 + rec) * 2 + p) * 256 + t * 128 + 32 * hh + mm) * 2 + (qf & 1);
+    base[0] = uint2{two(h[0], h[2]), two(h[1], h[3])};
+    base[128] = uint2{two(l[0], l[2]), two(l[1], l[3])};
+    if (stab) {
+        // of the operands' own values: their rounding then cancels between a
+        // code's products and the min's as far as the weight is small
+        float sum = 0.0f;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) sum += (float)h[u] + (float)l[u];
+        sum += __shfl_xor(sum, 1, 64);
+        sum += __shfl_xor(sum, 2, 64);
+        sum += __shfl_xor(sum, 4, 64);
+        if (qf == 0) {
+            const float s6 = __builtin_amdgcn_ldexpf(sum, -6);
+            const _Float16 sh = (_Float16)s6, sl = (_Float16)(s6 - (float)sh);
+            const uint32_t i = rec & 7, pos = (i & 4) | ((i & 1) << 1) | ((i >> 1) & 1);
+            _Float16* sp = (_Float16*)stab + (((size_t)ch * (nrec / 8) + rec / 8) * 128 + t * 64 + mm) * 8 + pos;
+            sp[0] = sh;
+            sp[32 * 8] = sl;
+        }
+    }
+}
 
 template <int MG, bool NORM = false, bool SUM = false, bool ATT = false>
 RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t K,
@@ -864,8 +909,9 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
             const uint32_t f = tid + T * i;
             f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
             if (m < M && f < nf) {
+                const uint32_t nsp = MG == 8 ? wide_splits(ps->full, ps->splits, 4 * f, 256, ps->nch, sch) : ps->splits;
                 t = *(const f32x4*)(ps->part + off + 4 * f);
-                for (uint32_t sp = 1; sp < ps->splits; ++sp) t += *(const f32x4*)(ps->part + off + sp * ss + 4 * f);
+                for (uint32_t sp = 1; sp < nsp; ++sp) t += *(const f32x4*)(ps->part + off + sp * ss + 4 * f);
                 if (ps->part2) {
                     f32x4 u = *(const f32x4*)(ps->part2 + off + 4 * f);
                     for (uint32_t sp = 1; sp < ps->splits; ++sp)
@@ -926,7 +972,7 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
 #pragma unroll
     for (uint32_t i = 0; i < NPT; ++i) {
         const uint32_t f = tid + T * i;
-        if (f >= nf) break;  // (the 8 lanes of a record share this)
+        if (f >= (MG == 8 ? nrec + (nrec & 1) : nrec) * 8) break;  // (the 8 lanes of a record share this)
         const uint32_t rec = f >> 3, qf = f & 7, kc = qf >> 1, half = qf & 1;
         const float xs[4] = {__builtin_amdgcn_ldexpf(v[i].x, -e), __builtin_amdgcn_ldexpf(v[i].y, -e),
                              __builtin_amdgcn_ldexpf(v[i].z, -e), __builtin_amdgcn_ldexpf(v[i].w, -e)};
@@ -935,6 +981,10 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
         for (int u = 0; u < 4; ++u) {
             h[u] = (_Float16)xs[u];
             l[u] = (_Float16)(xs[u] - (float)h[u]);
+        }
+        if constexpr (MG == 8) {
+            prep_store_wide(aops, stab, m, rec, qf, nrec, h, l);
+            continue;
         }
         // 16-byte entries 2·mm (hi) and 2·mm + 1 (lo) of k-group kc: this
         // float4 is their half `half`
@@ -960,6 +1010,7 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
 RT_GEMM_XH_PREP1(1)
 RT_GEMM_XH_PREP1(2)
 RT_GEMM_XH_PREP1(4)
+RT_GEMM_XH_PREP1(8)
 // the same preparation of RMSNorm(x)·γ, the normalised rows also written to
 // xn (when given)
 #define RT_GEMM_XH_PREP1N(MG)                                                                  \
@@ -971,6 +1022,7 @@ RT_GEMM_XH_PREP1(4)
 RT_GEMM_XH_PREP1N(1)
 RT_GEMM_XH_PREP1N(2)
 RT_GEMM_XH_PREP1N(4)
+RT_GEMM_XH_PREP1N(8)
 // the preparation of a row given as a GEMM's partial sums (PrepSum), plain or
 // RMS-normalised
 #define RT_GEMM_XH_PREP1S(MG)                                                                  \
@@ -988,6 +1040,11 @@ RT_GEMM_XH_PREP1N(4)
 RT_GEMM_XH_PREP1S(1)
 RT_GEMM_XH_PREP1S(2)
 RT_GEMM_XH_PREP1S(4)
+extern "C" __global__ void __launch_bounds__(1024) k_gemm_xh_prep1sn_mg8(
+    PrepSum ps, uint32_t M, uint32_t K, uint2* aops, int* etab, float* stab, const float* gamma,
+    float eps) {
+    gemm_xh_prep1_body<8, true, true>(nullptr, M, K, aops, etab, stab, gamma, eps, nullptr, &ps);
+}
 // the preparation of rows given as multi-query attention partials (PrepAttn)
 #define RT_GEMM_XH_PREP1A(MG)                                                                  \
     extern "C" __global__ void __launch_bounds__(1024) k_gemm_xh_prep1a_mg##MG(                \
@@ -998,6 +1055,7 @@ RT_GEMM_XH_PREP1S(4)
 RT_GEMM_XH_PREP1A(1)
 RT_GEMM_XH_PREP1A(2)
 RT_GEMM_XH_PREP1A(4)
+RT_GEMM_XH_PREP1A(8)
 RT_GEMM_XH_PREP(1)
 RT_GEMM_XH_PREP(2)
 RT_GEMM_XH_PREP(4)
@@ -1224,11 +1282,13 @@ RT_DEV void gemm3_body(const Gemm2Args& a, uint32_t bid = blockIdx.x, uint32_t n
 // the last split) cost ~9 µs of a 40 µs GEMM.
 extern "C" __global__ void __launch_bounds__(256) k_gemm_split_sum(const float* __restrict__ part, float* __restrict__ y,
                                                                  uint32_t M, uint32_t N, uint32_t splits,
-                                                                 uint32_t crow) {
+                                                                 uint32_t crow, uint32_t full, uint32_t tile) {
     // grid (⌈N / 1024⌉, M): thread → 4 consecutive outputs of row m
     const uint32_t m = blockIdx.y, n = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (n >= N) return;
     const uint32_t ch = m / crow, r = m % crow;
+    // (a wide GEMM's unsplit tiles are done)
+    if (full && wide_splits(full, 2, n, tile, (M + crow - 1) / crow, ch) == 1) return;
     const float* p = part + ((size_t)ch * splits * crow + r) * N + n;
     const size_t ss = (size_t)crow * N;
     if (n + 4 <= N && N % 4 == 0) {
@@ -1251,10 +1311,12 @@ extern "C" __global__ void __launch_bounds__(256) k_gemm_split_sum(const float* 
 //   res given:  Y = res + Y         (add_f32; Y may alias res).
 RT_DEV void split_sum_ep(const float* __restrict__ part, const float* __restrict__ part2, float* y,
                          uint32_t N, uint32_t splits, uint32_t crow,
-                         const uint16_t* __restrict__ bias, const float* res, uint32_t bx) {
+                         const uint16_t* __restrict__ bias, const float* res, uint32_t bx,
+                         uint32_t full, uint32_t tile, uint32_t nch) {
     const uint32_t m = blockIdx.y, n0 = (bx * 256 + threadIdx.x) * 4;
     if (n0 >= N) return;
     const uint32_t ch = m / crow, r = m % crow;
+    if (full && wide_splits(full, 2, n0, tile, nch, ch) == 1) return;  // done by the wide GEMM
     const size_t off = ((size_t)ch * splits * crow + r) * N, ss = (size_t)crow * N;
     if (N % 4 == 0 && (((uintptr_t)part | (uintptr_t)part2 | (uintptr_t)y | (uintptr_t)res) & 15) == 0 &&
         ((uintptr_t)bias & 7) == 0) {
@@ -1292,8 +1354,8 @@ RT_DEV void split_sum_ep(const float* __restrict__ part, const float* __restrict
 extern "C" __global__ void __launch_bounds__(256)
 k_gemm_split_sum_ep(const float* __restrict__ part, const float* __restrict__ part2, float* y,
                     uint32_t M, uint32_t N, uint32_t splits, uint32_t crow,
-                    const uint16_t* __restrict__ bias, const float* res) {
-    split_sum_ep(part, part2, y, N, splits, crow, bias, res, blockIdx.x);
+                    const uint16_t* __restrict__ bias, const float* res, uint32_t full, uint32_t tile) {
+    split_sum_ep(part, part2, y, N, splits, crow, bias, res, blockIdx.x, full, tile, (M + crow - 1) / crow);
 }
 // The split sums (+ bias) of up to three GEMMs of one set in one launch
 // (Q/K/V): workgroup columns [blk0[i], blk0[i + 1]) take output i.
@@ -1301,17 +1363,18 @@ struct EpSeg {
     const float* part;
     float* y;
     const uint16_t* bias;
-    uint32_t n, splits, blk0;
+    uint32_t n, splits, blk0, full;
 };
 struct EpSegs {
     EpSeg s[3];
-    uint32_t count, crow;
+    uint32_t count, crow, nch;
 };
 extern "C" __global__ void __launch_bounds__(256) k_gemm_split_sum_ep3(EpSegs a) {
     uint32_t i = 0;
     while (i + 1 < a.count && blockIdx.x >= a.s[i + 1].blk0) ++i;
     const EpSeg& g = a.s[i];
-    split_sum_ep(g.part, nullptr, g.y, g.n, g.splits, a.crow, g.bias, nullptr, blockIdx.x - g.blk0);
+    split_sum_ep(g.part, nullptr, g.y, g.n, g.splits, a.crow, g.bias, nullptr, blockIdx.x - g.blk0,
+                 g.full, 256, a.nch);
 }
 // k_gemm_split_sum_ep3 of the Q/K/V set with rope_kv_write_batch folded in:
 // segment 0 (q) rotated and written to q, segment 1 (k) rotated and written
@@ -1337,8 +1400,9 @@ extern "C" __global__ void __launch_bounds__(256) k_gemm_split_sum_qkv_rope(EpSe
     if (live) {
         const uint32_t ch = m / a.crow, r = m % a.crow;
         const size_t off = ((size_t)ch * g.splits * a.crow + r) * g.n, ss = (size_t)a.crow * g.n;
+        const uint32_t nsp = g.full ? wide_splits(g.full, g.splits, n0, 256, a.nch, ch) : g.splits;
         v = *(const f32x4*)(g.part + off + n0);
-        for (uint32_t sp = 1; sp < g.splits; ++sp) v += *(const f32x4*)(g.part + off + sp * ss + n0);
+        for (uint32_t sp = 1; sp < nsp; ++sp) v += *(const f32x4*)(g.part + off + sp * ss + n0);
         if (g.bias) {
             const uint2 b = *(const uint2*)(g.bias + n0);
             v += f32x4{h2f(b.x), h2f(b.x >> 16), h2f(b.y), h2f(b.y >> 16)};

@@ -277,6 +277,7 @@ struct rt_ctx {
     size_t max_lds = 65536;
     std::string err = "no error";
     bool capturing = false;
+    uint32_t gemm_wide_min = 32;  // RUNIT_GEMM_WIDE_MIN: rows above which a GEMM takes the wide form (A/B)
     bool gemm_direct = false;   // RUNIT_GEMM_DIRECT: force the unstaged GEMM kernel (tests)
     bool ksplit_enabled = true; // RUNIT_GEMV_KSPLIT=0: long K via the pre-pass instead (tests)
     // Workspace for activation records built by the long-K pre-pass; grows on
@@ -1330,6 +1331,7 @@ int rt_ctx_create(rt_ctx** out, const char* code_object_path) {
         c->max_lds = (size_t)lds;
     // A/B switches between the kernel bodies (tests and measurements)
     if (const char* g = getenv("RUNIT_GEMM_DIRECT")) c->gemm_direct = atoi(g) != 0;
+    if (const char* g = getenv("RUNIT_GEMM_WIDE_MIN")) c->gemm_wide_min = (uint32_t)atoi(g);
     if (const char* g = getenv("RUNIT_GEMM_F16")) c->gemm_f16 = atoi(g) != 0;
     if (const char* g = getenv("RUNIT_GEMM_W16")) c->gemm_w16 = atoi(g) != 0;
     if (const char* g = getenv("RUNIT_GEMM_Q6W8")) c->gemm_q6w8 = atoi(g);
@@ -1401,6 +1403,11 @@ int rt_ctx_create(rt_ctx** out, const char* code_object_path) {
         }
     names.push_back("k_act_limbs_rows_f32");
     names.push_back("k_act_limbs_rows_f32_q40");
+    for (const char* fm : kRowsFmts) names.push_back(std::string("k_gemmw_") + fm);
+    for (const char* fm : {"q8_0", "q4_0", "q4_0g", "q5_0", "q6k", "q6kg"})
+        names.push_back(std::string("k_gemmw_") + fm + "_o");
+    for (const char* v : {"", "n", "sn", "a"})
+        names.push_back(std::string("k_gemm_xh_prep1") + v + "_mg8");
     names.push_back("k_gemm3_q8_0_nb4_mg1");
     names.push_back("k_gemm3_q4_0_nb4_mg1");
     for (const char* b : kLsValuBases)
@@ -1930,8 +1937,9 @@ struct GemmFmt {
 // Y = the sum of the K splits' partial sums ([chunk][split][crow][N]),
 // in split order (k_gemm_split_sum).
 static int gemm_split_sum(rt_ctx* c, float* part, float* y, uint32_t m, uint32_t n, uint32_t splits,
-                          uint32_t crow) {
-    void* pp[] = {&part, &y, &m, &n, &splits, &crow};
+                          uint32_t crow, uint32_t full = 0) {
+    uint32_t tile = 256;  // of a wide GEMM, whose first `full` tiles are done
+    void* pp[] = {&part, &y, &m, &n, &splits, &crow, &full, &tile};
     return launch(c, "k_gemm_split_sum", dim3((n + 1023) / 1024, m), dim3(256), 0, pp);
 }
 
@@ -1942,14 +1950,99 @@ struct Gemm3Plan {
     uint64_t row_bytes;
     size_t a_bytes, e_bytes, s_bytes;  // prepared operands, row exponents, record sums
     size_t p_bytes;                    // K-split partial sums (splits > 1)
+    uint32_t full, quant;              // wide form: unsplit tiles, stages of a weight block
 };
+
+// Mirrors the device-side GemmWArgs / GemmWMulti (k_gemmw.hip).
+struct GemmWArgs {
+    const void* w;
+    const void* w2;
+    const void* aops;
+    const int* etab;
+    const void* ssum;
+    float* y;
+    float* part;
+    float* part2;
+    uint32_t M, N, nblk, nst, nchunks, splits, parts_all;
+    uint64_t row_bytes;
+    const uint16_t* bias;
+    const float* res;
+};
+struct GemmWMulti {
+    GemmWArgs a[3];
+    uint32_t t0[4];
+    uint32_t count, full, rem, splits, kst;
+};
+
+// Divides the tiles of the plans that share a wide launch over the grid: as
+// many whole rounds of resident workgroups as there are, and the remaining
+// tiles with K split so that they fill one more.  (All of a tile's K in one
+// workgroup otherwise: 1,184 tiles of the 7B gate and up at 512 rows on 512
+// resident workgroups took three rounds for 2.3 rounds of work.)
+static void gemmw_divide(const rt_ctx* c, Gemm3Plan* const* ps, uint32_t count) {
+    const Gemm3Plan& p0 = *ps[0];
+    uint32_t total = 0;
+    for (uint32_t i = 0; i < count; ++i) total += ps[i]->base;
+    const uint32_t nst = p0.nrec / 2, units = nst / p0.quant, rem = total % p0.cap;
+    uint32_t splits = 1;
+    // µs of one workgroup's tile at its share of the rate (about 1.7 TFLOP/s
+    // of hi + lo products each), 3 µs of start and end; a split tile's sums
+    // written and read at 4 TB/s, and 4 µs for the launch that adds them
+    const double t1 = nst * 64.0 * 65536.0 / 1.7e6;
+    double best = 1e30;
+    for (uint32_t sp = 1; sp <= std::min<uint32_t>(32, units) && rem; ++sp) {
+        const double rounds = (double)(((uint64_t)rem * sp + p0.cap - 1) / p0.cap);
+        const double t = rounds * (t1 / sp + 3.0) + (sp > 1 ? 4.0 + rem * sp * 2 * 65536.0 / 4e6 : 0.0);
+        if (t < best - 1e-9) { best = t; splits = sp; }
+    }
+    if (c->gemm_splits) splits = std::max(1u, std::min<uint32_t>(c->gemm_splits, units));
+    const uint32_t kst = (units + splits - 1) / splits * p0.quant;
+    splits = (nst + kst - 1) / kst;
+    uint32_t whole = splits == 1 ? total : total - rem;
+    for (uint32_t i = 0; i < count; ++i) {
+        Gemm3Plan& p = *ps[i];
+        p.full = std::min(whole, p.base);
+        whole -= p.full;
+        p.splits = p.full < p.base ? splits : 1;
+        p.kbs = kst;
+    }
+}
+
+// Plans the wide form (k_gemmw.hip; MG = 8 stands for its chunks of 64 rows)
+// of one matrix, or of a gate and up pair (pair: 128 rows of each a tile).
+// Any K that the preparation holds in registers.
+static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
+                       uint32_t k, Gemm3Plan& p, bool pair = false) {
+    if (m_rows <= c->gemm_wide_min || k > 20480 || !aligned(w, 16) || c->gemm_direct) return false;
+    p.nblk = k / f.blk_el;
+    const bool odd = p.nblk % 2 && !f.has_min;  // rows only 2-byte aligned
+    snprintf(p.kn, sizeof p.kn, odd ? "k_gemmw_%s_o" : "k_gemmw_%s", f.name);
+    p.waves = 4;
+    p.MG = 8;
+    p.nchunks = (m_rows + 63) / 64;
+    p.nrec = (k / 32 + 1) & ~1u;  // whole stages of two records
+    p.quant = f.blk_el / 64 ? f.blk_el / 64 : 1;
+    p.tiles = pair ? (n + 127) / 128 : (n + 255) / 256;
+    p.base = p.tiles * p.nchunks;
+    p.cap = (uint32_t)c->cu_count * std::min<uint32_t>(2, std::max<uint32_t>(1, occupancy(c, p.kn, 256, 0)));
+    p.row_bytes = (uint64_t)p.nblk * f.blk_bytes;
+    p.a_bytes = (size_t)p.nchunks * p.nrec * 8192;
+    p.e_bytes = (size_t)p.nchunks * 64 * sizeof(int);
+    p.s_bytes = f.has_min ? (size_t)p.nchunks * p.nrec * 256 : 0;
+    Gemm3Plan* one[] = {&p};
+    gemmw_divide(c, one, 1);
+    p.p_bytes = p.splits > 1 ? (size_t)p.splits * p.nchunks * 64 * n * sizeof(float) : 0;
+    return true;
+}
 
 // Plans the f16 form: 8 activation rows per group (MG ∈ {1, 2, 4}), hi/lo
 // f16 operands prepared by k_gemm_xh_prep*_mg*.  Returns kLsDecline where
 // the staged layout does not apply (the caller then takes the other forms).
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                       uint32_t k, Gemm3Plan& p) {
+    p = Gemm3Plan{};
     const uint32_t cu = (uint32_t)c->cu_count;
+    if (gemmw_plan(c, f, w, m_rows, n, k, p)) return RT_OK;
     const uint32_t groups = (m_rows + 7) / 8;
     const uint32_t MG = std::min<uint32_t>(f.max_mg_f16, groups <= 1 ? 1 : groups <= 2 ? 2 : 4);
     const uint32_t nchunks = (m_rows + 8 * MG - 1) / (8 * MG);
@@ -2092,6 +2185,42 @@ static int gemm3_prep(rt_ctx* c, const Gemm3Plan& p, const float* x, uint32_t m_
     return launch(c, pk, dim3(rows, parts), dim3(threads), 0, pp);
 }
 
+// One job of a wide launch over prepared operands: y for unsplit tiles (with
+// bias / res, or the SiLU product of a pair) unless parts_all, part (part2:
+// of w2) for the others.
+struct GemmWJob {
+    Gemm3Plan* p;
+    const void* w;
+    const void* w2;
+    const float* stab;
+    float* y;
+    float* part;
+    float* part2;
+    uint32_t n;
+    bool parts_all;
+    const uint16_t* bias;
+    const float* res;
+};
+static int gemmw_launch(rt_ctx* c, const GemmWJob* jobs, uint32_t count, const void* aops,
+                        const int* erow, uint32_t m_rows) {
+    GemmWMulti mm{};
+    mm.count = count;
+    mm.splits = 1;
+    for (uint32_t i = 0; i < count; ++i) {
+        const GemmWJob& j = jobs[i];
+        const Gemm3Plan& p = *j.p;
+        mm.a[i] = GemmWArgs{j.w, j.w2, aops, erow, j.stab, j.y, j.part, j.part2, m_rows, j.n, p.nblk,
+                            p.nrec / 2, p.nchunks, p.splits, j.parts_all, p.row_bytes, j.bias, j.res};
+        mm.t0[i + 1] = mm.t0[i] + p.base;
+        mm.full += p.full;
+        mm.rem += p.base - p.full;
+        mm.splits = std::max(mm.splits, p.splits);
+        mm.kst = p.kbs;
+    }
+    void* pp[] = {&mm};
+    return launch(c, jobs[0].p->kn, dim3(mm.full + mm.rem * mm.splits), dim3(256), 0, pp);
+}
+
 // The GEMM of a plan over prepared operands.  part: the partial sums
 // (splits > 1), left for the caller's sum when `leave_parts`; otherwise
 // summed here (k_gemm_split_sum, or in the GEMM with arrival counters).
@@ -2101,6 +2230,13 @@ static int gemm3_run(rt_ctx* c, const Gemm3Plan& p, const void* w, void* aops, i
                      float* stab, float* y, float* part, uint32_t m_rows, uint32_t n,
                      bool leave_parts = false, const uint16_t* bias = nullptr,
                      const float* res = nullptr) {
+    if (p.MG == 8) {
+        Gemm3Plan pw = p;
+        const GemmWJob j{&pw, w, nullptr, stab, y, part, nullptr, n, leave_parts, bias, res};
+        const int st = gemmw_launch(c, &j, 1, aops, erow, m_rows);
+        if (st != RT_OK || p.splits == 1 || leave_parts) return st;
+        return gemm_split_sum(c, part, y, m_rows, n, p.splits, 64, p.full);
+    }
     uint32_t cstride = 32;
     while (cstride > 1 && (size_t)p.base * cstride > kAttnCounters) cstride >>= 1;
     const bool sum_kernel = p.splits > 1 && (c->gemm_sum_kernel || leave_parts);
@@ -2408,17 +2544,18 @@ struct EpSeg {
     const float* part;
     float* y;
     const uint16_t* bias;
-    uint32_t n, splits, blk0;
+    uint32_t n, splits, blk0, full;
 };
 struct EpSegs {
     EpSeg s[3];
-    uint32_t count, crow;
+    uint32_t count, crow, nch;
 };
 
 static int gemm_split_sum_ep(rt_ctx* c, const float* part, const float* part2, float* y, uint32_t m,
                              uint32_t n, uint32_t splits, uint32_t crow, const uint16_t* bias,
-                             const float* res) {
-    void* pp[] = {(void*)&part, (void*)&part2, &y, &m, &n, &splits, &crow, (void*)&bias, (void*)&res};
+                             const float* res, uint32_t full = 0, uint32_t tile = 256) {
+    void* pp[] = {(void*)&part, (void*)&part2, &y, &m, &n, &splits, &crow, (void*)&bias, (void*)&res,
+                  &full, &tile};
     return launch(c, "k_gemm_split_sum_ep", dim3((n + 1023) / 1024, m), dim3(256), 0, pp);
 }
 
@@ -2429,6 +2566,95 @@ struct RopeKv {
     uint32_t head_dim, start_pos, max_seq;
     float theta;
 };
+
+// A GEMM set on the wide form: one preparation, the matrices of one format in
+// one launch (a SiLU pair as pairs of tiles whose product the GEMM stores),
+// then the sums of the tiles that split K; with `rope` every tile's sums go
+// through the partials to the launch that rotates and caches them.
+static int gemm_set_wide(rt_ctx* c, uint32_t count, const GemmFmt* const* f, Gemm3Plan* pl,
+                         const void* const* w, float* const* y, const uint32_t* n,
+                         const uint16_t* const* bias, const float* res, const float* x,
+                         uint32_t m_rows, uint32_t k, const float* gamma, float eps, float* xn,
+                         uint32_t silu_pair, const RopeKv* rope) {
+    const bool pair = silu_pair && f[0] == f[1] && gemmw_plan(c, *f[0], w[0], m_rows, n[0], k, pl[0], true);
+    const uint32_t mats = pair ? 1 : count;
+    // the matrices of one kernel (up to three) in one launch, divided together
+    uint32_t group[4], size[4] = {0, 0, 0, 0}, ngroups = 0;
+    for (uint32_t i = 0; i < mats; ++i) {
+        uint32_t g = ngroups;
+        for (uint32_t q = 0; q < i && c->gemm_multi; ++q)
+            if (strcmp(pl[q].kn, pl[i].kn) == 0 && size[group[q]] < 3) g = group[q];
+        group[i] = g;
+        ++size[g];
+        if (g == ngroups) ++ngroups;
+    }
+    for (uint32_t g = 0; g < ngroups; ++g) {
+        Gemm3Plan* ps[3];
+        uint32_t np = 0;
+        for (uint32_t i = 0; i < mats; ++i)
+            if (group[i] == g) ps[np++] = &pl[i];
+        gemmw_divide(c, ps, np);
+    }
+    const Gemm3Plan& p0 = pl[0];
+    bool any_min = false;
+    for (uint32_t i = 0; i < count; ++i) any_min |= f[i]->has_min;
+    const size_t s_bytes = any_min ? (size_t)p0.nchunks * p0.nrec * 256 : 0;
+    size_t total = p0.a_bytes + p0.e_bytes + s_bytes, poff[4], psize[4];
+    for (uint32_t i = 0; i < mats; ++i) {
+        poff[i] = total;
+        psize[i] = pl[i].splits > 1 || rope ? (size_t)pl[i].splits * p0.nchunks * 64 * n[i] * sizeof(float) : 0;
+        psize[i] = (psize[i] + 255) & ~(size_t)255;
+        total += pair ? 2 * psize[i] : psize[i];
+    }
+    int st = ensure_ws(c, total, "gemm_set");
+    if (st != RT_OK) return st;
+    char* ws = (char*)c->ws;
+    int* erow = (int*)(ws + p0.a_bytes);
+    float* stab = s_bytes ? (float*)(ws + p0.a_bytes + p0.e_bytes) : nullptr;
+    st = gemm3_prep(c, p0, x, m_rows, k, ws, erow, stab, gamma, eps, gamma ? xn : nullptr);
+    auto part = [&](uint32_t i) { return psize[i] ? (float*)(ws + poff[i]) : nullptr; };
+    for (uint32_t g = 0; g < ngroups && st == RT_OK; ++g) {
+        GemmWJob jobs[3];
+        uint32_t nj = 0;
+        for (uint32_t i = 0; i < mats; ++i)
+            if (group[i] == g)
+                jobs[nj++] = GemmWJob{&pl[i], w[i], pair ? w[1] : nullptr, f[i]->has_min ? stab : nullptr,
+                                      y[i], part(i), pair ? (float*)(ws + poff[i] + psize[i]) : nullptr,
+                                      n[i], rope != nullptr, bias ? bias[i] : nullptr, res};
+        st = gemmw_launch(c, jobs, nj, ws, erow, m_rows);
+    }
+    if (st != RT_OK) return st;
+    if (pair)
+        return pl[0].splits == 1 ? RT_OK
+                                 : gemm_split_sum_ep(c, part(0), (float*)(ws + poff[0] + psize[0]), y[0],
+                                                     m_rows, n[0], pl[0].splits, 64, nullptr, nullptr,
+                                                     pl[0].full, 128);
+    EpSegs es{};
+    es.crow = 64;
+    es.nch = p0.nchunks;
+    for (uint32_t i = 0; i < mats; ++i) {
+        if (!psize[i]) continue;
+        const uint16_t* b = bias ? bias[i] : nullptr;
+        if (res || count > 3) {
+            st = gemm_split_sum_ep(c, part(i), nullptr, y[i], m_rows, n[i], pl[i].splits, 64, b, res, pl[i].full);
+            if (st != RT_OK) return st;
+            continue;
+        }
+        EpSeg& g = es.s[es.count];
+        g = EpSeg{part(i), y[i], b, n[i], pl[i].splits,
+                  es.count ? es.s[es.count - 1].blk0 + (es.s[es.count - 1].n + 1023) / 1024 : 0, pl[i].full};
+        ++es.count;
+    }
+    if (es.count) {
+        const EpSeg& g = es.s[es.count - 1];
+        RopeKv rk = rope ? *rope : RopeKv{};
+        void* pp[] = {&es, &rk};
+        st = launch(c, rope ? "k_gemm_split_sum_qkv_rope" : "k_gemm_split_sum_ep3",
+                    dim3(g.blk0 + (g.n + 1023) / 1024, m_rows), dim3(256), 0, pp);
+    }
+    if (st != RT_OK || !silu_pair) return st;
+    return rt_silu_mul_f32(c, y[0], y[1], y[0], m_rows * n[0]);
+}
 
 // rt_gemm_set_f32; with `rope` (count 3: q, k, v) the sums also rotate q and
 // k and write k and v to the caches (k_gemm_split_sum_qkv_rope), or, on the
@@ -2508,6 +2734,9 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
                                               m_rows, rope->max_seq);
         return RT_OK;
     }
+    if (pl[0].MG == 8)
+        return gemm_set_wide(c, count, f, pl, w, y, n, bias, res, x, m_rows, k, gamma, eps, xn,
+                             silu_pair, rope);
     // workspace: [operands | row exponents | record sums | partials of each matrix]
     bool any_min = false;
     for (uint32_t i = 0; i < count; ++i) any_min |= f[i]->has_min;
@@ -2626,7 +2855,7 @@ struct PrepSum {
     const float* part2;
     const float* res;
     float* y;
-    uint32_t splits, crow;
+    uint32_t splits, crow, full, nch;
 };
 
 // Mirrors the device-side PrepAttn (k_gemm.hip).
@@ -2690,8 +2919,9 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     if (st == RT_OK) st = gemm3_plan(c, *fg, w_gate, m_rows, ff, h, pg);
     if (st == RT_OK) st = gemm3_plan(c, *fu, w_up, m_rows, ff, h, pu);
     if (st == RT_OK) st = gemm3_plan(c, *fd, w_down, m_rows, h, ff, pd);
-    if (st == kLsDecline || (st == RT_OK && (pg.MG != po.MG || pu.MG != po.MG || pd.MG != po.MG ||
-                                             pg.splits != pu.splits)))
+    if (st == kLsDecline ||
+        (st == RT_OK && (pg.MG != po.MG || pu.MG != po.MG || pd.MG != po.MG ||
+                         (po.MG == 8 ? fg != fu : pg.splits != pu.splits))))
         return plan_only ? RT_OK : sets();
     if (st != RT_OK) return st;
     if (plan_only) {
@@ -2702,10 +2932,16 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     // of the SiLU product (K = ff), then the partial sums of O, gate, up, down
     const uint32_t MG = po.MG, nch = po.nchunks, crow = 8 * MG;
     auto ops = [&](uint32_t k, bool mins) {
-        const size_t a = (size_t)nch * (k / 32) * MG * 64 * 16, e = (size_t)nch * 8 * MG * sizeof(int);
-        const size_t sb = mins ? (size_t)nch * (k / 32) * 8 * MG * sizeof(float) : 0;
+        // (the wide form pads an odd number of records)
+        const size_t nrec = MG == 8 ? (k / 32 + 1) & ~1u : k / 32;
+        const size_t a = (size_t)nch * nrec * MG * 64 * 16, e = (size_t)nch * 8 * MG * sizeof(int);
+        const size_t sb = mins ? (size_t)nch * nrec * 8 * MG * sizeof(float) : 0;
         return std::array<size_t, 3>{a, e, sb};
     };
+    if (MG == 8) {  // gate and up as pairs of tiles of one launch
+        gemmw_plan(c, *fg, w_gate, m_rows, ff, h, pg, true);
+        pu.splits = pg.splits;
+    }
     auto parts = [&](const Gemm3Plan& p, uint32_t n) {
         return (size_t)std::max<uint32_t>(1, p.splits) * nch * crow * n * sizeof(float);
     };
@@ -2749,13 +2985,30 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     char pk[48];
     uint32_t M = m_rows, K = h;
     {
-        PrepSum ps{part_o, nullptr, x, x_mid, po.splits, crow};
+        PrepSum ps{part_o, nullptr, x, x_mid, po.splits, crow, po.full, nch};
         void* aops = at(3);
         int* erow = (int*)at(4);
         float* stab = (float*)at(5);
         snprintf(pk, sizeof pk, "k_gemm_xh_prep1sn_mg%u", MG);
         void* pp[] = {&ps, &M, &K, &aops, &erow, &stab, (void*)&gamma, &eps};
         st = launch(c, pk, dim3(nch * 8 * MG), dim3(1024), 0, pp);
+    }
+    if (st == RT_OK && MG == 8) {
+        // the product silu(gate)·up from the GEMM (the tiles that split K
+        // from their sums), prepared for down; x = x_mid + down the same way
+        const GemmWJob gu{&pg, w_gate, w_up, fg->has_min ? (float*)at(5) : nullptr, g, part_g, part_u,
+                          ff, false, nullptr, nullptr};
+        st = gemmw_launch(c, &gu, 1, at(3), (int*)at(4), m_rows);
+        if (st == RT_OK && pg.splits > 1)
+            st = gemm_split_sum_ep(c, part_g, part_u, g, m_rows, ff, pg.splits, 64, nullptr, nullptr,
+                                   pg.full, 128);
+        if (st == RT_OK) st = gemm3_prep(c, pd, g, m_rows, ff, at(6), (int*)at(7), (float*)at(8));
+        const GemmWJob dn{&pd, w_down, nullptr, fd->has_min ? (float*)at(8) : nullptr, x, part_d, nullptr,
+                          h, false, nullptr, x_mid};
+        if (st == RT_OK) st = gemmw_launch(c, &dn, 1, at(6), (int*)at(7), m_rows);
+        if (st == RT_OK && pd.splits > 1)
+            st = gemm_split_sum_ep(c, part_d, nullptr, x, m_rows, h, pd.splits, 64, nullptr, x_mid, pd.full);
+        return st;
     }
     // gate and up (one launch where they share a kernel), their partials
     // left; silu(Σ gate)·Σ up prepared for down
@@ -2769,7 +3022,7 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     if (m_rows >= c->gemm_block_silu_min) {
         // the SiLU sum in the preparation (one workgroup per row reads the
         // row's partials of gate and up)
-        PrepSum ps{part_g, part_u, nullptr, nullptr, pg.splits, crow};
+        PrepSum ps{part_g, part_u, nullptr, nullptr, pg.splits, crow, 0, nch};
         void* aops = at(6);
         int* erow = (int*)at(7);
         float* stab = (float*)at(8);

@@ -1,0 +1,126 @@
+"""The wide batched GEMM (k_gemmw_<fmt>, more than 32 activation rows) of every
+block format against the oracle's per-row f64 GEMV of the same packed blocks,
+at the edges of its tiles: rows around one and two 64-row chunks, weight rows
+around 256-row tiles, K of one block, of an odd number of blocks, of one and
+several super-blocks, and K ranges split over workgroups.  Tolerance: every
+output within 1e-4·Σ|w·x| (gpu_helpers); the form's own error is the 22 bits
+of the f16 pairs and some ten f32 roundings, below 1e-6·Σ|w·x|, checked too."""
+import numpy as np
+import pytest
+
+import oracle_lib as ora
+import test_gpu_gemm_set
+from runit_mac_amd import dispatch as d
+from gpu_helpers import check_close, device_weights
+from test_gpu_fused import ffn_check
+
+pytestmark = pytest.mark.gpu
+
+SMALL = ("q8_0", "q4_0", "q4_0g", "q5_0")
+SUPER = ("q4k", "q4kg", "q5k", "q5kg", "q6k", "q6kg")
+
+
+def _check(ctx, fmt, m, n, k, seed):
+    w, raw = device_weights(ctx, fmt, n, k, seed)
+    rng = np.random.default_rng(seed)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[m // 2] *= 1e-3  # rows of their own scale, and an all-zero one
+    x[m - 1] = 0.0
+    y = ctx.new_buffer(4 * (m * n + 64))
+    y.write(np.full(m * n + 64, 7.0, np.float32))
+    getattr(d, f"gemm_{fmt}_f32")(ctx, w, ctx.buffer_from(x), y, m, n, k)
+    odd = "_o" if (k // d.BLOCK[fmt][0]) % 2 and fmt not in ("q4k", "q4kg", "q5k", "q5kg") else ""
+    assert d.last_launch_name(ctx) in (f"k_gemmw_{fmt}{odd}", "k_gemm_split_sum")
+    ctx.flush()
+    got = y.read(np.float32, m * n + 64)
+    assert np.all(got[m * n:] == 7.0), "past the last row"
+    ref, sabs = ora.gemv(fmt, raw, x, n, k)
+    check_close(got[:m * n], ref.ravel(), sabs.ravel(), f"{fmt} {m}x{n}x{k}")
+    err = np.abs(got[:m * n].astype(np.float64) - ref.ravel())
+    assert np.all(err <= 1e-6 * sabs.ravel()), f"{fmt} {m}x{n}x{k}: {(err / np.maximum(sabs.ravel(), 1e-30)).max():.2e}"
+
+
+@pytest.mark.parametrize("fmt", SMALL)
+@pytest.mark.parametrize("m,n,k", [(33, 1, 32), (64, 257, 96), (65, 300, 2080), (130, 511, 896)])
+def test_wide_gemm_block_formats(ctx, fmt, m, n, k):
+    _check(ctx, fmt, m, n, k, 900 + m)
+
+
+@pytest.mark.parametrize("fmt", SUPER)
+@pytest.mark.parametrize("m,n,k", [(33, 3, 256), (64, 257, 768), (129, 300, 4096)])
+def test_wide_gemm_super_block_formats(ctx, fmt, m, n, k):
+    _check(ctx, fmt, m, n, k, 920 + m)
+
+
+@pytest.mark.parametrize("fmt", ["q8_0", "q4kg"])
+def test_wide_gemm_whole_and_split_tiles(ctx, fmt):
+    """520 tiles: 512 of one workgroup each and 8 with K split (256 compute
+    units of two workgroups each), the last one ragged."""
+    _check(ctx, fmt, 33, 256 * 519 + 5, 512, 940)
+
+
+@pytest.mark.parametrize("fmts", [("q4k", "q4k", "q6k"), ("q8_0", "q8_0", "q8_0")])
+def test_wide_set_bias(ctx, fmts):
+    test_gpu_gemm_set.test_gemm_set_qkv_norm_bias(ctx, fmts, 70)
+
+
+@pytest.mark.parametrize("fmt,m", [("q4k", 33), ("q8_0", 70)])
+def test_wide_set_silu_pair(ctx, fmt, m):
+    test_gpu_gemm_set.test_gemm_set_silu_pair(ctx, fmt, m)
+
+
+@pytest.mark.parametrize("fmt,n,k", [("q6k", 1024, 2048), ("q8_0", 896, 4864), ("q4_0", 1000, 928)])
+def test_wide_set_residual(ctx, fmt, n, k):
+    test_gpu_gemm_set.test_gemm_set_residual(ctx, fmt, n, k, 70)
+
+
+def test_wide_set_of_four_and_mixed_pair(ctx):
+    """Four matrices of one format (two launches), and a SiLU pair of two
+    formats (separate products)."""
+    m, h, n = 70, 1024, 300
+    x = np.random.default_rng(5).standard_normal((m, h)).astype(np.float32)
+    xb = ctx.buffer_from(x)
+    W = [device_weights(ctx, "q4k", n, h, 960 + i) for i in range(4)]
+    ys = [ctx.new_buffer(4 * m * n) for _ in range(4)]
+    d.gemm_set_f32(ctx, ["q4k"] * 4, [w for w, _ in W], ys, [n] * 4, xb, m, h)
+    ctx.flush()
+    for y, (_, raw) in zip(ys, W):
+        ref, sabs = ora.gemv("q4k", raw, x, n, h)
+        check_close(y.read(np.float32, m * n), ref.ravel(), sabs.ravel(), "set of four")
+    w8, raw8 = device_weights(ctx, "q8_0", n, h, 970)
+    d.gemm_set_f32(ctx, ["q4k", "q8_0"], [W[0][0], w8], ys[:2], [n, n], xb, m, h, silu_pair=True)
+    ctx.flush()
+    g, gs = ora.gemv("q4k", W[0][1], x, n, h)
+    u, us = ora.gemv("q8_0", raw8, x, n, h)
+    ffn_check(ys[0].read(np.float32, m * n), g.ravel(), gs.ravel(), u.ravel(), us.ravel(), "mixed pair")
+
+
+def test_wide_qkv_rope_equals_set_then_rope(ctx):
+    """As test_gemm_qkv_rope_equals_set_then_rope, at 70 rows: q and keys to
+    2e-6 of their range (fused multiply-adds may contract differently), values
+    exactly."""
+    m, h, hd, heads, kvh, S, start = 70, 1024, 64, 14, 2, 128, 20
+    qd, kvd, fmts = heads * hd, kvh * hd, ("q4kg", "q4kg", "q6kg")
+    W = [device_weights(ctx, f, n, h, 980 + i)[0] for i, (f, n) in enumerate(zip(fmts, (qd, kvd, kvd)))]
+    rng = np.random.default_rng(7)
+    x = ctx.buffer_from(rng.standard_normal((m, h)).astype(np.float32))
+    gamma = ctx.buffer_from((1 + 0.1 * rng.standard_normal(h)).astype(np.float32))
+    biases = [ctx.buffer_from((0.1 * rng.standard_normal(n)).astype(np.float16).view(np.uint16))
+              for n in (qd, kvd, kvd)]
+    cache0 = rng.standard_normal(kvh * S * hd).astype(np.float32)
+    outs = []
+    for fused in (True, False):
+        q, k, v = (ctx.new_buffer(4 * m * n) for n in (qd, kvd, kvd))
+        xn, kc, vc = ctx.new_buffer(4 * m * h), ctx.buffer_from(cache0), ctx.buffer_from(cache0)
+        if fused:
+            d.gemm_qkv_rope_f32(ctx, fmts, *W, *biases, x, gamma, 1e-6, xn, q, k, v, kc, vc, m, h,
+                                qd, kvd, hd, start, 10000.0, S)
+        else:
+            d.gemm_set_f32(ctx, list(fmts), W, [q, k, v], [qd, kvd, kvd], x, m, h, biases=biases,
+                           gamma=gamma, eps=1e-6, xn=xn)
+            d.rope_kv_write_batch_f32(ctx, q, k, v, kc, vc, hd, heads, kvh, start, 10000.0, m, S)
+        ctx.flush()
+        outs.append([b.read(np.float32, n) for b, n in ((q, m * qd), (kc, cache0.size), (vc, cache0.size))])
+    for a, b, what in zip(outs[0][:2], outs[1][:2], ("q", "k cache")):
+        assert np.max(np.abs(a - b)) <= 2e-6 * np.abs(b).max(), what
+    assert np.array_equal(outs[0][2], outs[1][2]), "v cache"
