@@ -6,7 +6,7 @@
 // A workgroup's tile is 256 weight rows × 64 activation rows: four waves of 64
 // weight rows each, all 64 activation rows.  The activations, prepared as f16
 // pairs hi + lo in MFMA order (prep_store_wide, k_gemm.hip), go from memory
-// straight to LDS, two stages of 64 elements of K double-buffered; every wave
+// straight to LDS in stages of 64 elements of K; every wave
 // reads all of a stage, one read feeding two v_mfma_f32_32x32x16_f16.  The
 // weights need no LDS: each lane loads its own weight row's bytes and decodes
 // them to the operand it feeds, once per 64 activation rows (the 32-row tiles
@@ -17,8 +17,10 @@
 // operations; without its weight loads the kernel runs at 1.05-1.13 PFLOP/s of
 // them at 512×16384×4096, a large f16 product of the library at 1.2.  With
 // them: Q4_K 840 TFLOP/s, Q4_0 870, Q8_0 750, Q6_K 720 (preparation included;
-// k_gemm3_*: 350-490).  Measured and not taken: loads two stages ahead (four
-// LDS buffers, partial waits): Q8_0 183 → 187 µs, Q4_K 153 → 157.
+// k_gemm3_*: 350-490).  A lone workgroup on a CU is bound by its waves' own
+// chain (1.3 µs a stage), which the loads two stages ahead keep fed: Q8_0
+// 64×3584×3584 26.2 → 24.2 µs, Q6_K 37×3584×18944 60.5 → 55.4 against loads
+// one stage ahead; with two workgroups on every CU the two are level.
 #include <type_traits>
 #include "rt_formats.h"
 #include "rt_shared.h"
@@ -103,6 +105,8 @@ RT_DEV void both_halves(uint32_t v, uint32_t& lo, uint32_t& hi) {
     lo = r[0];
     hi = r[1];
 }
+// Of a format: Q, stages of a block (1: blocks of 32); LU, stages that one
+// load() covers; LOADS, the fewest load instructions it can compile to.
 // A lane's weight row: a wave-uniform base and the lane's 32-bit offset, so
 // that the loads take a scalar base and no 64-bit vector arithmetic
 struct Row {
@@ -112,7 +116,7 @@ struct Row {
 struct NoSh {};
 template <bool OA>
 struct WQ8_0T {
-    static constexpr uint32_t BLK_BYTES = 34, U = 2, LU = 1;
+    static constexpr uint32_t BLK_BYTES = 34, Q = 1, LU = 1, LOADS = OA ? 5 : 8;
     static constexpr bool CHAIN = false, HALF = false, TAIL = false;
     struct Raw {
         u32x4 q[2];
@@ -167,7 +171,7 @@ struct WQ8_0T {
 // j + 16; reference layout: byte i holds elements 2i and 2i + 1.
 template <bool G, bool OA>
 struct WQ4_0T {
-    static constexpr uint32_t BLK_BYTES = 18, U = 2, LU = 1;
+    static constexpr uint32_t BLK_BYTES = 18, Q = 1, LU = 1, LOADS = OA ? 4 : 8;
     static constexpr bool CHAIN = false, HALF = false, TAIL = false;
     struct Raw {
         uint32_t q[2][2], e;
@@ -240,7 +244,7 @@ RT_DEV u32x4 spread_bits(uint32_t b, uint32_t at) {
 }
 template <bool OA>
 struct WQ5_0T {  // value d·(q − 16); bit j of qh is the fifth bit of element j
-    static constexpr uint32_t BLK_BYTES = 22, U = 2, LU = 1;
+    static constexpr uint32_t BLK_BYTES = 22, Q = 1, LU = 1, LOADS = OA ? 6 : 12;
     static constexpr bool CHAIN = false, HALF = false, TAIL = false;
     struct Raw {
         uint32_t q[2][2], e, f;
@@ -330,7 +334,7 @@ struct KQ {
 };
 template <bool G>
 struct WQ4KT {
-    static constexpr uint32_t BLK_BYTES = 144, U = 4, LU = 1;
+    static constexpr uint32_t BLK_BYTES = 144, Q = 4, LU = 1, LOADS = 2;
     static constexpr int MID = 8;  // centre of the codes
     static constexpr bool CHAIN = true, HALF = false, TAIL = false;
     struct Raw {
@@ -360,7 +364,7 @@ struct WQ4KT {
 };
 template <bool G>
 struct WQ5KT {
-    static constexpr uint32_t BLK_BYTES = 176, U = 4, LU = 1;
+    static constexpr uint32_t BLK_BYTES = 176, Q = 4, LU = 1, LOADS = 4;
     static constexpr int MID = 16;  // centre of the codes
     static constexpr bool CHAIN = true, HALF = false, TAIL = false;
     struct Raw {
@@ -428,7 +432,7 @@ struct WQ5KT {
 // register, the last piece's from Sh.
 template <bool G, bool OA>
 struct WQ6KT {
-    static constexpr uint32_t BLK_BYTES = 210, U = 4, LU = 2;
+    static constexpr uint32_t BLK_BYTES = 210, Q = 4, LU = 2, LOADS = OA ? 8 : 6;
     static constexpr bool CHAIN = false, HALF = G, TAIL = true;
     struct Raw {
         u32x4 l[2], h;
@@ -544,10 +548,25 @@ typedef __attribute__((address_space(3))) void* lptr_t;
 
 RT_DEV float silu_mul(float g, float u) { return g / (1.0f + expf(-g)) * u; }
 
+// Waits until at most VM of the wave's vector memory operations (they complete
+// in order) and none of its LDS operations are under way, then for the
+// workgroup.
+template <int VM>
+RT_DEV void wait_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((VM & 15) | (VM >> 4) << 14 | 7 << 4);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
+// Pipeline: while stage s is computed, the activations of stage s + 2 go to LDS
+// (one of three buffers) and, once the weights of stage s are decoded, those
+// of stage s + 2 to their registers; the wait at the end of a stage leaves
+// both under way.
 template <class P>
 RT_DEV void gemmw_tile(const GemmWArgs& a, uint32_t t, uint32_t split, uint32_t st0, uint32_t st1,
                        bool whole, u32x4 (*lds)[1024]) {
-    constexpr int NT = 2, MT = 2;
+    constexpr int NT = 2, MT = 2, LU = P::LU;
     const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t j = lane & 31, h = lane >> 5;
     // chunks fastest: the workgroups of one tile of weights run together
@@ -591,40 +610,52 @@ RT_DEV void gemmw_tile(const GemmWArgs& a, uint32_t t, uint32_t split, uint32_t 
     if constexpr (P::CHAIN) load_hdr(hdr, st0);
     if constexpr (P::TAIL) PT::load_tail(tl_nx, rowx, st0);
     P::load(raw[0], sh[0], row, rowx, st0, h, a.nblk);
-    __syncthreads();
+    stage_in(min(st0 + 1, st1 - 1), 1);
+    if constexpr (LU == 1) P::load(raw[1], sh[1], row, rowx, min(st0 + 1, st1 - 1), h, a.nblk);
+    wait_barrier<0>();
     if constexpr (P::TAIL) PT::spread_tail(tl_nx, tl);
+    uint32_t buf = 0;  // of the stage
     auto stage = [&](uint32_t st, auto us_) {
-        constexpr int US = decltype(us_)::value, LU = P::LU, RB = (US / LU) & 1;
-        const uint32_t nx = min(st + 1, st1 - 1);
-        stage_in(nx, (US + 1) & 1);
-        if constexpr ((US + 1) % LU == 0) {
-            constexpr int NB = ((US + 1) / LU) & 1;
-            P::load(raw[NB], sh[NB], row, rowx, nx, h, a.nblk);
+        constexpr int US = decltype(us_)::value, RB = (US / LU) & 1;
+        const uint32_t nx = min(st + 2, st1 - 1);
+        stage_in(nx, buf == 0 ? 2 : buf - 1);
+        if constexpr (LU == 2 && US % 2 == 0) P::load(raw[RB ^ 1], sh[RB ^ 1], row, rowx, nx, h, a.nblk);
+        if constexpr (P::CHAIN && US == 1) {
+#pragma unroll
+            for (int t = 0; t < MT; ++t)
+                sm[t] = __builtin_bit_cast(h8_t, a.ssum[((size_t)ch * (a.nst / 4) + st / 4) * 128 + t * 64 + lane]);
         }
-        if constexpr (P::CHAIN && US == 3) load_hdr(hdr_nx, nx);
-        if constexpr (P::TAIL && US == 3) PT::load_tail(tl_nx, rowx, nx);
-        __builtin_amdgcn_sched_barrier(0);  // the next stage's loads go out first
+        if constexpr (P::CHAIN && US == 2) load_hdr(hdr_nx, nx);
+        if constexpr (P::TAIL && US == 2) PT::load_tail(tl_nx, rowx, nx);
+        __builtin_amdgcn_sched_barrier(0);  // these loads go out first
         if constexpr (US % LU == 0) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) P::arrange(raw[RB][nt], sh[RB], nt, st, h);
         }
-        const u32x4* ab = lds[US & 1];
+        h8_t B[NT][2][2];
+        float sc[NT][2][2];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+            if constexpr (P::CHAIN) {
+                P::template pair<US>(raw[RB][nt], hdr[nt], h, B[nt]);
+                sc[nt][0][0] = h2f(hdr[nt].x);
+            } else {
+#pragma unroll
+                for (int rr = 0; rr < 2; ++rr) {
+                    if constexpr (P::TAIL) P::template rec<US>(raw[RB][nt], tl[nt], rr, B[nt][rr], sc[nt][rr]);
+                    else P::template rec<US>(raw[RB][nt], rr, h, B[nt][rr], sc[nt][rr]);
+                }
+            }
+        }
+        if constexpr (LU == 1) P::load(raw[RB], sh[RB], row, rowx, nx, h, a.nblk);
+        // (an odd number of stages: the last is left out, but not its loads and
+        // waits, so that every wait counts one path)
+        const bool live = P::Q == 4 || US == 0 || st < st1;
+        const u32x4* ab = lds[buf];
         auto A = [&](int rr, int p, int t, int hl) {
             return __builtin_bit_cast(h8_t, ab[(((rr * 2 + p) * 2 + t) * 2 + hl) * 64 + lane]);
         };
         if constexpr (P::CHAIN) {
-            if (US == 2) {
-#pragma unroll
-                for (int t = 0; t < MT; ++t)
-                    sm[t] = __builtin_bit_cast(h8_t, a.ssum[((size_t)ch * (a.nst / 4) + st / 4) * 128 + t * 64 + lane]);
-            }
-            h8_t B[NT][2][2];
-            float d[NT];
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                P::template pair<US>(raw[RB][nt], hdr[nt], h, B[nt]);
-                d[nt] = h2f(hdr[nt].x);
-            }
 #pragma unroll
             for (int rr = 0; rr < 2; ++rr)
 #pragma unroll
@@ -658,57 +689,54 @@ RT_DEV void gemmw_tile(const GemmWArgs& a, uint32_t t, uint32_t split, uint32_t 
 #pragma unroll
                     for (int t = 0; t < MT; ++t) {
 #pragma unroll
-                        for (int i = 0; i < 16; ++i) acc[nt][t][i] = __builtin_fmaf(d[nt], C[nt][t][i], acc[nt][t][i]);
+                        for (int i = 0; i < 16; ++i) acc[nt][t][i] = __builtin_fmaf(sc[nt][0][0], C[nt][t][i], acc[nt][t][i]);
                         C[nt][t] = f16v{};
                     }
             }
-        } else {
+        } else if (live) {
 #pragma unroll
-            for (int rr = 0; rr < 2; ++rr) {
-                h8_t B[NT][2];
-                float sc[NT][2];
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) {
-                    if constexpr (P::TAIL) P::template rec<US>(raw[RB][nt], tl[nt], rr, B[nt], sc[nt]);
-                    else P::template rec<US>(raw[RB][nt], rr, h, B[nt], sc[nt]);
-                }
+            for (int rr = 0; rr < 2; ++rr)
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
                     const h8_t a0 = A(rr, 0, t, 0), a1 = A(rr, 0, t, 1), a2 = A(rr, 1, t, 0), a3 = A(rr, 1, t, 1);
 #pragma unroll
                     for (int nt = 0; nt < NT; ++nt) {
-                        f16v c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, B[nt][0], f16v{}, 0, 0, 0);
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, B[nt][0], c, 0, 0, 0);
+                        const h8_t b0 = B[nt][rr][0], b1 = B[nt][rr][1];
+                        f16v c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a0, b0, f16v{}, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a1, b0, c, 0, 0, 0);
                         if (P::HALF) {
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) acc[nt][t][i] = __builtin_fmaf(sc[nt][0], c[i], acc[nt][t][i]);
+                            for (int i = 0; i < 16; ++i)
+                                acc[nt][t][i] = __builtin_fmaf(sc[nt][rr][0], c[i], acc[nt][t][i]);
                             c = f16v{};
                         }
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, B[nt][1], c, 0, 0, 0);
-                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a3, B[nt][1], c, 0, 0, 0);
-                        const float s = sc[nt][P::HALF ? 1 : 0];
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a2, b1, c, 0, 0, 0);
+                        c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a3, b1, c, 0, 0, 0);
+                        const float s = sc[nt][rr][P::HALF ? 1 : 0];
 #pragma unroll
                         for (int i = 0; i < 16; ++i) acc[nt][t][i] = __builtin_fmaf(s, c[i], acc[nt][t][i]);
                     }
                 }
-            }
         }
-        __syncthreads();
+        // everything issued before this stage's loads has arrived
+        wait_barrier<4 + (LU == 1 || US % 2 == 0 ? (int)P::LOADS : 0)>();
         __builtin_amdgcn_sched_barrier(0);  // (uses of the loads stay behind their wait)
         if constexpr (P::CHAIN && US == 3) {
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) hdr[nt] = hdr_nx[nt];
         }
         if constexpr (P::TAIL && US == 3) PT::spread_tail(tl_nx, tl);
+        buf = buf == 2 ? 0 : buf + 1;
     };
-    for (uint32_t st = st0; st < st1; st += P::U) {
+    for (uint32_t st = st0; st < st1; st += P::Q == 4 ? 4 : 2) {
         stage(st, std::integral_constant<int, 0>{});
-        if (P::U == 4 || st + 1 < st1) stage(st + 1, std::integral_constant<int, 1>{});
-        if constexpr (P::U == 4) {
+        stage(st + 1, std::integral_constant<int, 1>{});
+        if constexpr (P::Q == 4) {
             stage(st + 2, std::integral_constant<int, 2>{});
             stage(st + 3, std::integral_constant<int, 3>{});
         }
     }
+    __builtin_amdgcn_s_waitcnt(0);  // no load to LDS outlives the workgroup
     // lane l holds row 8(i / 4) + 4h + i % 4 of a tile of activation rows for
     // weight row l % 32; the activation rows' exponents scale the sums
     const uint32_t m0 = ch * 64 + 4 * h;
@@ -773,7 +801,7 @@ RT_DEV uint32_t xcd_order(uint32_t b, uint32_t n) {
 }
 template <class P>
 RT_DEV void gemmw_body(const GemmWMulti& m) {
-    __shared__ u32x4 lds[2][1024];
+    __shared__ u32x4 lds[3][1024];
     const bool whole = blockIdx.x < m.full;
     uint32_t t, split = 0;
     if (whole) {

@@ -277,6 +277,10 @@ struct rt_ctx {
     size_t max_lds = 65536;
     std::string err = "no error";
     bool capturing = false;
+    // RUNIT_GEMM_WIDE_WORK: rows × weights from which a call takes the wide form (A/B).  Below,
+    // its tiles leave the grid to K splits: Q8_0 64×3584×3584 (0.8e9) 24.2 against 22.6 µs,
+    // 300×4864×1024 (1.5e9) 30 / 25, 128×3584×3584 (1.6e9) 28.5 / 32.7, 33×18944×3584 (2.2e9) 40 / 57
+    uint64_t gemm_wide_work = 1600000000ull;
     uint32_t gemm_wide_min = 32;  // RUNIT_GEMM_WIDE_MIN: rows above which a GEMM takes the wide form (A/B)
     bool gemm_direct = false;   // RUNIT_GEMM_DIRECT: force the unstaged GEMM kernel (tests)
     bool ksplit_enabled = true; // RUNIT_GEMV_KSPLIT=0: long K via the pre-pass instead (tests)
@@ -1331,6 +1335,7 @@ int rt_ctx_create(rt_ctx** out, const char* code_object_path) {
         c->max_lds = (size_t)lds;
     // A/B switches between the kernel bodies (tests and measurements)
     if (const char* g = getenv("RUNIT_GEMM_DIRECT")) c->gemm_direct = atoi(g) != 0;
+    if (const char* g = getenv("RUNIT_GEMM_WIDE_WORK")) c->gemm_wide_work = strtoull(g, nullptr, 10);
     if (const char* g = getenv("RUNIT_GEMM_WIDE_MIN")) c->gemm_wide_min = (uint32_t)atoi(g);
     if (const char* g = getenv("RUNIT_GEMM_F16")) c->gemm_f16 = atoi(g) != 0;
     if (const char* g = getenv("RUNIT_GEMM_W16")) c->gemm_w16 = atoi(g) != 0;
@@ -1983,16 +1988,23 @@ static void gemmw_divide(const rt_ctx* c, Gemm3Plan* const* ps, uint32_t count) 
     const Gemm3Plan& p0 = *ps[0];
     uint32_t total = 0;
     for (uint32_t i = 0; i < count; ++i) total += ps[i]->base;
-    const uint32_t nst = p0.nrec / 2, units = nst / p0.quant, rem = total % p0.cap;
+    const uint32_t nst = p0.nrec / 2, rem = total % p0.cap;
+    const uint32_t units = (nst + p0.quant - 1) / p0.quant;
     uint32_t splits = 1;
-    // µs of one workgroup's tile at its share of the rate (about 1.7 TFLOP/s
-    // of hi + lo products each), 3 µs of start and end; a split tile's sums
-    // written and read at 4 TB/s, and 4 µs for the launch that adds them
-    const double t1 = nst * 64.0 * 65536.0 / 1.7e6;
+    // µs of `wgs` workgroups of `stages` stages: 1.3 a stage with one
+    // workgroup on a CU, 2.6 with two, and 3 of start and end (Q8_0 64×3584×
+    // 3584 at 2 / 4 splits 37 / 21 µs, 512×16384×4096 175 µs in 64 stages).
+    // Split tiles: a launch of about 5 µs that adds them, their sums written
+    // and read.
+    const uint32_t cu = (uint32_t)c->cu_count;
+    auto run_us = [&](uint64_t wgs, uint32_t stages) {
+        const uint64_t rounds = wgs / p0.cap, last = wgs % p0.cap;
+        return rounds * (2.6 * stages + 3.0) + (last > cu ? 2.6 * stages + 3.0 : last ? 1.3 * stages + 3.0 : 0.0);
+    };
     double best = 1e30;
     for (uint32_t sp = 1; sp <= std::min<uint32_t>(32, units) && rem; ++sp) {
-        const double rounds = (double)(((uint64_t)rem * sp + p0.cap - 1) / p0.cap);
-        const double t = rounds * (t1 / sp + 3.0) + (sp > 1 ? 4.0 + rem * sp * 2 * 65536.0 / 4e6 : 0.0);
+        const uint32_t stages = (units + sp - 1) / sp * p0.quant;
+        const double t = run_us((uint64_t)rem * sp, stages) + (sp > 1 ? 5.0 + rem * sp * 0.022 : 0.0);
         if (t < best - 1e-9) { best = t; splits = sp; }
     }
     if (c->gemm_splits) splits = std::max(1u, std::min<uint32_t>(c->gemm_splits, units));
@@ -2021,7 +2033,7 @@ static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_ro
     p.MG = 8;
     p.nchunks = (m_rows + 63) / 64;
     p.nrec = (k / 32 + 1) & ~1u;  // whole stages of two records
-    p.quant = f.blk_el / 64 ? f.blk_el / 64 : 1;
+    p.quant = f.blk_el / 64 ? f.blk_el / 64 : 2;  // (the kernel's stages go in pairs)
     p.tiles = pair ? (n + 127) / 128 : (n + 255) / 256;
     p.base = p.tiles * p.nchunks;
     p.cap = (uint32_t)c->cu_count * std::min<uint32_t>(2, std::max<uint32_t>(1, occupancy(c, p.kn, 256, 0)));
@@ -2038,11 +2050,14 @@ static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_ro
 // Plans the f16 form: 8 activation rows per group (MG ∈ {1, 2, 4}), hi/lo
 // f16 operands prepared by k_gemm_xh_prep*_mg*.  Returns kLsDecline where
 // the staged layout does not apply (the caller then takes the other forms).
+// work: rows × weights of the whole call (0: of this matrix).  The wide form
+// takes calls of gemm_wide_work on, and those whose K the stages here do not tile.
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
-                      uint32_t k, Gemm3Plan& p) {
+                      uint32_t k, Gemm3Plan& p, uint64_t work = 0) {
     p = Gemm3Plan{};
     const uint32_t cu = (uint32_t)c->cu_count;
-    if (gemmw_plan(c, f, w, m_rows, n, k, p)) return RT_OK;
+    if (!work) work = (uint64_t)m_rows * n * k;
+    if (work >= c->gemm_wide_work && gemmw_plan(c, f, w, m_rows, n, k, p)) return RT_OK;
     const uint32_t groups = (m_rows + 7) / 8;
     const uint32_t MG = std::min<uint32_t>(f.max_mg_f16, groups <= 1 ? 1 : groups <= 2 ? 2 : 4);
     const uint32_t nchunks = (m_rows + 8 * MG - 1) / (8 * MG);
@@ -2063,7 +2078,7 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     }
     const uint32_t seg = NB * f.blk_bytes, vb = seg % 16 == 0 ? 16 : (seg % 8 == 0 ? 8 : 4);
     if (nblk % NB != 0 || !aligned(w, 16) || row_bytes % vb != 0 || c->gemm_direct)
-        return kLsDecline;
+        return gemmw_plan(c, f, w, m_rows, n, k, p) ? RT_OK : kLsDecline;
     // Q6_K: 128-row tiles with one operand and one weight buffer
     const bool q6 = f.blk_bytes == 210;
     const bool w8ok = !q6 || (c->gemm_q6w8 >> (MG == 4 ? 0 : MG == 2 ? 1 : 2) & 1);
@@ -2702,12 +2717,16 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
                   (!rope || (aligned(y[0], 16) && aligned(rope->kc, 16) && aligned(rope->vc, 16))) &&
                   (!rope || (1024 % rope->head_dim == 0 && rope->head_dim % 4 == 0 && rope->head_dim <= 512 && n[0] % 4 == 0 && n[1] % 4 == 0 &&
                              c->gemm_rope));
+    uint64_t work = 0;
+    for (uint32_t i = 0; i < count; ++i) work += (uint64_t)m_rows * n[i] * k;
+    for (uint32_t i = 0; shared && i < count; ++i) shared = !bias || aligned(bias[i], 8);
     for (uint32_t i = 0; shared && i < count; ++i) {
-        if (bias && bias[i] && !aligned(bias[i], 8)) {
-            shared = false;
-            break;
+        int st = gemm3_plan(c, *f[i], w[i], m_rows, n[i], k, pl[i], work);
+        if (st == RT_OK && i && pl[i].MG != pl[0].MG && (pl[i].MG == 8 || pl[0].MG == 8) && work != UINT64_MAX) {
+            work = UINT64_MAX;  // one of them only has the wide form
+            i = UINT32_MAX;
+            continue;
         }
-        const int st = gemm3_plan(c, *f[i], w[i], m_rows, n[i], k, pl[i]);
         if (st != RT_OK && st != kLsDecline) return st;
         shared = st == RT_OK && pl[i].MG == pl[0].MG;
     }
@@ -2915,10 +2934,16 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         qd % fo->blk_el || h % fg->blk_el || h % fu->blk_el || ff % fd->blk_el)
         return plan_only ? RT_OK : sets();
     Gemm3Plan po, pg, pu, pd;
-    int st = gemm3_plan(c, *fo, w_o, m_rows, h, qd, po);
-    if (st == RT_OK) st = gemm3_plan(c, *fg, w_gate, m_rows, ff, h, pg);
-    if (st == RT_OK) st = gemm3_plan(c, *fu, w_up, m_rows, ff, h, pu);
-    if (st == RT_OK) st = gemm3_plan(c, *fd, w_down, m_rows, h, ff, pd);
+    auto plan = [&](uint64_t work) {
+        int s = gemm3_plan(c, *fo, w_o, m_rows, h, qd, po, work);
+        if (s == RT_OK) s = gemm3_plan(c, *fg, w_gate, m_rows, ff, h, pg, work);
+        if (s == RT_OK) s = gemm3_plan(c, *fu, w_up, m_rows, ff, h, pu, work);
+        if (s == RT_OK) s = gemm3_plan(c, *fd, w_down, m_rows, h, ff, pd, work);
+        return s;
+    };
+    int st = plan((uint64_t)m_rows * h * (qd + 3ull * ff));
+    if (st == RT_OK && (po.MG == 8 || pg.MG == 8 || pu.MG == 8 || pd.MG == 8))
+        st = plan(UINT64_MAX);  // (one of them may only have the wide form)
     if (st == kLsDecline ||
         (st == RT_OK && (pg.MG != po.MG || pu.MG != po.MG || pd.MG != po.MG ||
                          (po.MG == 8 ? fg != fu : pg.splits != pu.splits))))

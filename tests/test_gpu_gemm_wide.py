@@ -5,6 +5,8 @@ around 256-row tiles, K of one block, of an odd number of blocks, of one and
 several super-blocks, and K ranges split over workgroups.  Tolerance: every
 output within 1e-4·Σ|w·x| (gpu_helpers); the form's own error is the 22 bits
 of the f16 pairs and some ten f32 roundings, below 1e-6·Σ|w·x|, checked too."""
+import os
+
 import numpy as np
 import pytest
 
@@ -15,6 +17,20 @@ from gpu_helpers import check_close, device_weights
 from test_gpu_fused import ffn_check
 
 pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    """A context whose calls take the wide form from 33 rows on, however small
+    (by default from 1.6e9 rows × weights on, and where no other form fits)."""
+    os.environ["RUNIT_GEMM_WIDE_WORK"] = "0"
+    try:
+        c = d.HipContext()
+    finally:
+        del os.environ["RUNIT_GEMM_WIDE_WORK"]
+    yield c
+    c.close()
+
 
 SMALL = ("q8_0", "q4_0", "q4_0g", "q5_0")
 SUPER = ("q4k", "q4kg", "q5k", "q5kg", "q6k", "q6kg")
