@@ -19,6 +19,7 @@
 // operand order ([chunk][block][group][lane] 8-byte entries, one coalesced
 // dwordx2 per lane) plus the block exponents ([chunk][block][mm][group]).
 #include "rt_formats.h"
+#include "rt_gemm.h"
 #include "rt_shared.h"
 
 typedef long i64_t;
@@ -784,92 +785,6 @@ RT_DEV void gemm_xh_prep_body(const float* __restrict__ x, uint32_t M, uint32_t 
 // (thread t: float4s t, t + 1024, ...), reduces the row's largest |x|, then
 // writes each float4 as half of a 16-byte A entry (hi, lo) — one round trip
 // to memory instead of three.
-// The row of a preparation given as the K-split partial sums of the GEMM
-// that produced it ([chunk][split][crow][K], as k_gemm_split_sum reads
-// them): x = Σ part (SILU: silu(Σ part)·Σ part2), then res + x; written to y
-// when given.
-struct PrepSum {
-    const float* part;
-    const float* part2;
-    const float* res;
-    float* y;
-    uint32_t splits, crow;
-    uint32_t full, nch;  // wide GEMM: its first `full` tiles are unsplit (wide_splits)
-};
-
-// p[0] + p[ss] + ... (splits terms, in order), four loads in flight (a loop
-// that waited for each took 8.7 µs at 16 splits of 37×3584)
-RT_DEV f32x4 split_add(const float* __restrict__ p, size_t ss, uint32_t splits) {
-    f32x4 v = *(const f32x4*)p, t1, t2, t3;
-    for (uint32_t sp = 1; sp < splits; sp += 4) {
-        const uint32_t r = splits - sp;
-        const float* q = p + sp * ss;
-        const f32x4 t0 = *(const f32x4*)q;
-        if (r > 1) t1 = *(const f32x4*)(q + ss);
-        if (r > 2) t2 = *(const f32x4*)(q + 2 * ss);
-        if (r > 3) t3 = *(const f32x4*)(q + 3 * ss);
-        v += t0;
-        if (r > 1) v += t1;
-        if (r > 2) v += t2;
-        if (r > 3) v += t3;
-    }
-    return v;
-}
-
-// K splits of the 256-column tile that holds column n of chunk ch in the
-// partial sums of a wide GEMM (k_gemmw.hip): tiles in the order [column tile]
-// [chunk], the first `full` of them unsplit.
-RT_DEV uint32_t wide_splits(uint32_t full, uint32_t splits, uint32_t n, uint32_t tile, uint32_t nch, uint32_t ch) {
-    return n / tile * nch + ch < full ? 1 : splits;
-}
-
-// The row of a preparation given as the split partials of the multi-query
-// attention (k_attn_mq_f32_hd*, parts-only, one sequence): element (head h,
-// d) of row r is column qi = r·G + h mod G of KV head h / G, merged over the
-// nsp key ranges as that kernel's last workgroup merges them.
-struct PrepAttn {
-    const float* part;
-    const float* ml;
-    uint32_t nsp, G, hd, cgs;
-};
-
-// One float4 of the operands of k_gemmw.hip (chunks of 64 rows): [chunk]
-// [stage of 2 records][record][MFMA p][32-row tile][hi, lo][64 lanes] entries
-// of 8 halves; lane 32·h + row holds elements 16p + 8h .. + 7 of the record in
-// the order 0 2 1 3 4 6 5 7.  A record past K is zero.  stab: the record sums
-// of each super-block as f16 pairs hi + lo of Σx·2^-6, [chunk][super-block]
-// [tile][32·(hi, lo) + row][8 records in the same order].
-RT_DEV void prep_store_wide(uint2* __restrict__ aops, float* __restrict__ stab, uint32_t m,
-                            uint32_t rec, uint32_t qf, uint32_t nrec, const _Float16 (&h)[4],
-                            const _Float16 (&l)[4]) {
-    auto two = [](_Float16 a, _Float16 b) {
-        return (uint32_t)__builtin_bit_cast(uint16_t, a) | ((uint32_t)__builtin_bit_cast(uint16_t, b) << 16);
-    };
-    const uint32_t ch = m / 64, t = m / 32 % 2, mm = m % 32;
-    const uint32_t p = qf >> 2, hh = (qf >> 1) & 1;
-    uint2* base = aops + ((((size_t)ch * ((nrec + 1) / 2) * 2 + rec) * 2 + p) * 256 + t * 128 + 32 * hh + mm) * 2 + (qf & 1);
-    base[0] = uint2{two(h[0], h[2]), two(h[1], h[3])};
-    base[128] = uint2{two(l[0], l[2]), two(l[1], l[3])};
-    if (stab) {
-        // of the operands' own values: their rounding then cancels between a
-        // code's products and the min's as far as the weight is small
-        float sum = 0.0f;
-#pragma unroll
-        for (int u = 0; u < 4; ++u) sum += (float)h[u] + (float)l[u];
-        sum += __shfl_xor(sum, 1, 64);
-        sum += __shfl_xor(sum, 2, 64);
-        sum += __shfl_xor(sum, 4, 64);
-        if (qf == 0) {
-            const float s6 = __builtin_amdgcn_ldexpf(sum, -6);
-            const _Float16 sh = (_Float16)s6, sl = (_Float16)(s6 - (float)sh);
-            const uint32_t i = rec & 7, pos = (i & 4) | ((i & 1) << 1) | ((i >> 1) & 1);
-            _Float16* sp = (_Float16*)stab + (((size_t)ch * (nrec / 8) + rec / 8) * 128 + t * 64 + mm) * 8 + pos;
-            sp[0] = sh;
-            sp[32 * 8] = sl;
-        }
-    }
-}
-
 template <int MG, bool NORM = false, bool SUM = false, bool ATT = false>
 RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t K,
                                uint2* __restrict__ aops, int* __restrict__ etab,
@@ -928,8 +843,7 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
             const uint32_t f = tid + T * i;
             f32x4 t = {0.0f, 0.0f, 0.0f, 0.0f};
             if (m < M && f < nf) {
-                const uint32_t nsp = MG == 8 ? wide_splits(ps->full, ps->splits, 4 * f, 256, ps->nch, sch) : ps->splits;
-                t = split_add(ps->part + off + 4 * f, ss, nsp);
+                t = split_add(ps->part + off + 4 * f, ss, ps->splits);
                 if (ps->part2) {
                     const f32x4 u = split_add(ps->part2 + off + 4 * f, ss, ps->splits);
                     t = f32x4{t.x / (1.0f + expf(-t.x)) * u.x, t.y / (1.0f + expf(-t.y)) * u.y,
@@ -988,7 +902,7 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
 #pragma unroll
     for (uint32_t i = 0; i < NPT; ++i) {
         const uint32_t f = tid + T * i;
-        if (f >= (MG == 8 ? nrec + (nrec & 1) : nrec) * 8) break;  // (the 8 lanes of a record share this)
+        if (f >= nf) break;  // (the 8 lanes of a record share this)
         const uint32_t rec = f >> 3, qf = f & 7, kc = qf >> 1, half = qf & 1;
         const float xs[4] = {__builtin_amdgcn_ldexpf(v[i].x, -e), __builtin_amdgcn_ldexpf(v[i].y, -e),
                              __builtin_amdgcn_ldexpf(v[i].z, -e), __builtin_amdgcn_ldexpf(v[i].w, -e)};
@@ -997,10 +911,6 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
         for (int u = 0; u < 4; ++u) {
             h[u] = (_Float16)xs[u];
             l[u] = (_Float16)(xs[u] - (float)h[u]);
-        }
-        if constexpr (MG == 8) {
-            prep_store_wide(aops, stab, m, rec, qf, nrec, h, l);
-            continue;
         }
         // 16-byte entries 2·mm (hi) and 2·mm + 1 (lo) of k-group kc: this
         // float4 is their half `half`
@@ -1026,7 +936,6 @@ RT_DEV void gemm_xh_prep1_body(const float* __restrict__ x, uint32_t M, uint32_t
 RT_GEMM_XH_PREP1(1)
 RT_GEMM_XH_PREP1(2)
 RT_GEMM_XH_PREP1(4)
-RT_GEMM_XH_PREP1(8)
 // the same preparation of RMSNorm(x)·γ, the normalised rows also written to
 // xn (when given)
 #define RT_GEMM_XH_PREP1N(MG)                                                                  \
@@ -1038,7 +947,6 @@ RT_GEMM_XH_PREP1(8)
 RT_GEMM_XH_PREP1N(1)
 RT_GEMM_XH_PREP1N(2)
 RT_GEMM_XH_PREP1N(4)
-RT_GEMM_XH_PREP1N(8)
 // the preparation of a row given as a GEMM's partial sums (PrepSum), plain or
 // RMS-normalised
 #define RT_GEMM_XH_PREP1S(MG)                                                                  \
@@ -1056,11 +964,6 @@ RT_GEMM_XH_PREP1N(8)
 RT_GEMM_XH_PREP1S(1)
 RT_GEMM_XH_PREP1S(2)
 RT_GEMM_XH_PREP1S(4)
-extern "C" __global__ void __launch_bounds__(1024) k_gemm_xh_prep1sn_mg8(
-    PrepSum ps, uint32_t M, uint32_t K, uint2* aops, int* etab, float* stab, const float* gamma,
-    float eps) {
-    gemm_xh_prep1_body<8, true, true>(nullptr, M, K, aops, etab, stab, gamma, eps, nullptr, &ps);
-}
 // the preparation of rows given as multi-query attention partials (PrepAttn)
 #define RT_GEMM_XH_PREP1A(MG)                                                                  \
     extern "C" __global__ void __launch_bounds__(1024) k_gemm_xh_prep1a_mg##MG(                \
@@ -1071,7 +974,6 @@ extern "C" __global__ void __launch_bounds__(1024) k_gemm_xh_prep1sn_mg8(
 RT_GEMM_XH_PREP1A(1)
 RT_GEMM_XH_PREP1A(2)
 RT_GEMM_XH_PREP1A(4)
-RT_GEMM_XH_PREP1A(8)
 RT_GEMM_XH_PREP(1)
 RT_GEMM_XH_PREP(2)
 RT_GEMM_XH_PREP(4)

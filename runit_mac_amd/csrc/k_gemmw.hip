@@ -5,7 +5,7 @@
 //
 // A workgroup's tile is 256 weight rows × 64 activation rows: four waves of 64
 // weight rows each, all 64 activation rows.  The activations, prepared as f16
-// pairs hi + lo in MFMA order (prep_store_wide, k_gemm.hip), go from memory
+// pairs hi + lo in MFMA order (prep_row below), go from memory
 // straight to LDS in stages of 64 elements of K; every wave
 // reads all of a stage, one read feeding two v_mfma_f32_32x32x16_f16.  The
 // weights need no LDS: each lane loads its own weight row's bytes and decodes
@@ -23,6 +23,7 @@
 // one stage ahead; with two workgroups on every CU the two are level.
 #include <type_traits>
 #include "rt_formats.h"
+#include "rt_gemm.h"
 #include "rt_shared.h"
 
 typedef _Float16 h2_t __attribute__((ext_vector_type(2)));
@@ -817,6 +818,190 @@ RT_DEV void gemmw_body(const GemmWMulti& m) {
     const uint32_t st0 = whole ? 0 : split * m.kst, st1 = whole ? nst : min(nst, st0 + m.kst);
     gemmw_tile<P>(m.a[i], t - m.t0[i], split, st0, st1, whole, lds);
 }
+// ───────────────────────────── activation preparation ─────────────────────────────
+//
+// A workgroup per (padded) row holds the row in registers, thread u + T·i the
+// elements 8u .. 8u + 7, scales it by the power of two e that takes its
+// largest |x| into [2^14, 2^15) and writes hi = f16(x·2^-e) and lo =
+// f16(x·2^-e − hi): [chunk of 64 rows][stage][record][MFMA p][32-row tile]
+// [hi, lo][lane 32h + row] entries of 8 halves, elements 16p + 8h .. + 7 of the
+// record in the order 0 2 1 3 4 6 5 7.  Rows past M and a record past K are
+// zero.  ssum: the record sums of each super-block as f16 pairs hi + lo of
+// Σx·2^-6, [chunk][super-block][tile][32·(hi, lo) + row][8 records, same order].
+//
+// Bound: memory.  Eight rows share each 128-byte line of the operands, so
+// consecutive rows go to one XCD (xcd_order), whose L2 joins their writes.
+enum PrepMode { kPrepRows, kPrepNorm, kPrepSumNorm, kPrepAttn };
+struct PrepWArgs {
+    const float* x;      // rows (kPrepRows, kPrepNorm)
+    const float* gamma;  // RMSNorm of the row first (kPrepNorm, kPrepSumNorm): x·rsqrt(mean(x²) + eps)·γ
+    float* xn;           // kPrepNorm: the normalised rows, when given
+    u32x4* aops;
+    int* etab;
+    _Float16* ssum;      // or null
+    uint32_t M, K;
+    float eps;
+    PrepSum ps;          // kPrepSumNorm
+    PrepAttn pa;         // kPrepAttn
+};
+template <int T>
+RT_DEV float wg_reduce(float v, float* red, bool max) {
+    for (int o = 32; o > 0; o >>= 1) {
+        const float w = __shfl_xor(v, o, 64);
+        v = max ? fmaxf(v, w) : v + w;
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    float r = red[0];
+#pragma unroll
+    for (int w = 1; w < T / 64; ++w) r = max ? fmaxf(r, red[w]) : r + red[w];
+    return r;
+}
+template <int T, int NPT, PrepMode MODE>
+RT_DEV void prep_row(const PrepWArgs& a) {
+    __shared__ float red[2][T / 64];
+    const uint32_t m = xcd_order(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const uint32_t nu = a.K / 8, nup = (a.K / 32 + 1) / 2 * 8;  // with the zero record
+    const bool row = m < a.M;
+    f32x4 v[NPT][2];
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+        const uint32_t u = tid + T * i;
+        v[i][0] = v[i][1] = f32x4{0, 0, 0, 0};
+        if (!row || u >= nu) continue;
+        if constexpr (MODE == kPrepSumNorm) {
+            const PrepSum& ps = a.ps;
+            const uint32_t ch = m / 64;
+            const size_t off = ((size_t)ch * ps.splits * 64 + m % 64) * a.K + 8 * u, ss = (size_t)64 * a.K;
+            const uint32_t nsp = wide_splits(ps.full, ps.splits, 8 * u, 256, ps.nch, ch);
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                v[i][q] = *(const f32x4*)(ps.res + (size_t)m * a.K + 8 * u + 4 * q) +
+                          split_add(ps.part + off + 4 * q, ss, nsp);
+                *(f32x4*)(ps.y + (size_t)m * a.K + 8 * u + 4 * q) = v[i][q];
+            }
+        } else if constexpr (MODE == kPrepAttn) {
+            // element (head, d) of the row, merged over the nsp key ranges as
+            // the attention's last workgroup merges them
+            const PrepAttn& pa = a.pa;
+            const float NEG = -__builtin_huge_valf();
+            const uint32_t h = 8 * u / pa.hd, d = 8 * u % pa.hd, kvh = h / pa.G;
+            const uint32_t qi = m * pa.G + h % pa.G, cg = qi / 16, col = qi % 16;
+            const size_t pair = (size_t)kvh * pa.cgs + cg;
+            const float* mlv = pa.ml + (pair * pa.nsp * 16 + col) * 2;
+            float mj[RT_ATTN_MQ_NSP_MAX], lj[RT_ATTN_MQ_NSP_MAX];
+            f32x4 pj[RT_ATTN_MQ_NSP_MAX][2];
+#pragma unroll
+            for (uint32_t j = 0; j < RT_ATTN_MQ_NSP_MAX; ++j) {
+                const uint32_t jj = j < pa.nsp ? j : 0;
+                mj[j] = mlv[32 * jj];
+                lj[j] = mlv[32 * jj + 1];
+                const f32x4* pp = (const f32x4*)(pa.part + ((pair * pa.nsp + jj) * 16 + col) * pa.hd + d);
+                pj[j][0] = pp[0];
+                pj[j][1] = pp[1];
+            }
+            float Mx = NEG, L = 0.0f;
+#pragma unroll
+            for (uint32_t j = 0; j < RT_ATTN_MQ_NSP_MAX; ++j) Mx = fmaxf(Mx, mj[j]);
+            f32x4 o[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+            for (uint32_t j = 0; j < RT_ATTN_MQ_NSP_MAX; ++j) {
+                const float w = (j >= pa.nsp || mj[j] == NEG) ? 0.0f : expf(mj[j] - Mx);
+                L += w * lj[j];
+                o[0] += w * pj[j][0];
+                o[1] += w * pj[j][1];
+            }
+            v[i][0] = o[0] / L;
+            v[i][1] = o[1] / L;
+        } else {
+            const f32x4* xr = (const f32x4*)(a.x + (size_t)m * a.K + 8 * u);
+            v[i][0] = xr[0];
+            v[i][1] = xr[1];
+        }
+    }
+    if constexpr (MODE == kPrepNorm || MODE == kPrepSumNorm) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int i = 0; i < NPT; ++i)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const f32x4 t = v[i][q];
+                ss += t.x * t.x + t.y * t.y + t.z * t.z + t.w * t.w;
+            }
+        const float rms = rsqrtf(wg_reduce<T>(ss, red[0], false) / (float)a.K + a.eps);
+#pragma unroll
+        for (int i = 0; i < NPT; ++i) {
+            const uint32_t u = tid + T * i;
+            if (!row || u >= nu) continue;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const f32x4 g = *(const f32x4*)(a.gamma + 8 * u + 4 * q), t = v[i][q];
+                v[i][q] = f32x4{t.x * rms * g.x, t.y * rms * g.y, t.z * rms * g.z, t.w * rms * g.w};
+                if (MODE == kPrepNorm && a.xn) *(f32x4*)(a.xn + (size_t)m * a.K + 8 * u + 4 * q) = v[i][q];
+            }
+        }
+    }
+    float mx = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NPT; ++i)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const f32x4 t = v[i][q];
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(t.x), fabsf(t.y)), fmaxf(fabsf(t.z), fabsf(t.w))));
+        }
+    mx = wg_reduce<T>(mx, red[1], true);
+    const int e = mx > 0.0f ? __builtin_amdgcn_frexp_expf(mx) - 15 : 0;
+    if (tid == 0) a.etab[m] = e;
+    const uint32_t ch = m / 64, t32 = m / 32 % 2, mm = m % 32;
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+        const uint32_t u = tid + T * i;
+        if (u >= nup) break;  // (the four lanes of a record share this)
+        _Float16 h[8], l[8];
+        float sum = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float xs = __builtin_amdgcn_ldexpf(v[i][j / 4][j % 4], -e);
+            h[j] = (_Float16)xs;
+            l[j] = (_Float16)(xs - (float)h[j]);
+            sum += (float)h[j] + (float)l[j];
+        }
+        const uint32_t rec = u >> 2, p = (u >> 1) & 1, hh = u & 1;
+        u32x4* base = a.aops + (((size_t)ch * (nup / 4) + rec) * 2 + p) * 256 + t32 * 128 + 32 * hh + mm;
+        auto two = [](_Float16 x, _Float16 y) {
+            return (uint32_t)__builtin_bit_cast(uint16_t, x) | ((uint32_t)__builtin_bit_cast(uint16_t, y) << 16);
+        };
+        base[0] = u32x4{two(h[0], h[2]), two(h[1], h[3]), two(h[4], h[6]), two(h[5], h[7])};
+        base[64] = u32x4{two(l[0], l[2]), two(l[1], l[3]), two(l[4], l[6]), two(l[5], l[7])};
+        if (a.ssum) {
+            // of the operands' own values: their rounding then cancels between a
+            // code's products and the min's as far as the weight is small
+            sum += __shfl_xor(sum, 1, 64);
+            sum += __shfl_xor(sum, 2, 64);
+            if ((u & 3) == 0) {
+                const float s6 = __builtin_amdgcn_ldexpf(sum, -6);
+                const _Float16 sh = (_Float16)s6, sl = (_Float16)(s6 - (float)sh);
+                const uint32_t r = rec & 7, pos = (r & 4) | ((r & 1) << 1) | ((r >> 1) & 1);
+                _Float16* sp = a.ssum + (((size_t)ch * (nup / 32) + rec / 8) * 128 + t32 * 64 + mm) * 8 + pos;
+                sp[0] = sh;
+                sp[32 * 8] = sl;
+            }
+        }
+    }
+}
+// 256 threads up to K = 4096, 1024 up to 20,480 (24,576)
+#define RT_GEMMW_PREP(FN, MODE)                                                               \
+    extern "C" __global__ void __launch_bounds__(256) k_gemmw_prep##FN(PrepWArgs a) {         \
+        prep_row<256, 2, MODE>(a);                                                            \
+    }                                                                                         \
+    extern "C" __global__ void __launch_bounds__(1024) k_gemmw_prep##FN##_l(PrepWArgs a) {    \
+        prep_row<1024, 3, MODE>(a);                                                           \
+    }
+RT_GEMMW_PREP(, kPrepRows)
+RT_GEMMW_PREP(_n, kPrepNorm)
+RT_GEMMW_PREP(_sn, kPrepSumNorm)
+RT_GEMMW_PREP(_a, kPrepAttn)
+
 #define RT_GEMMW(FN, ...)                                                                     \
     extern "C" __global__ void __launch_bounds__(256, 2) k_gemmw_##FN(GemmWMulti m) {         \
         gemmw_body<__VA_ARGS__>(m);                                                           \

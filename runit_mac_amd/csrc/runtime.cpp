@@ -1411,8 +1411,8 @@ int rt_ctx_create(rt_ctx** out, const char* code_object_path) {
     for (const char* fm : kRowsFmts) names.push_back(std::string("k_gemmw_") + fm);
     for (const char* fm : {"q8_0", "q4_0", "q4_0g", "q5_0", "q6k", "q6kg"})
         names.push_back(std::string("k_gemmw_") + fm + "_o");
-    for (const char* v : {"", "n", "sn", "a"})
-        names.push_back(std::string("k_gemm_xh_prep1") + v + "_mg8");
+    for (const char* v : {"", "_n", "_sn", "_a"})
+        for (const char* l : {"", "_l"}) names.push_back(std::string("k_gemmw_prep") + v + l);
     names.push_back("k_gemm3_q8_0_nb4_mg1");
     names.push_back("k_gemm3_q4_0_nb4_mg1");
     for (const char* b : kLsValuBases)
@@ -2165,6 +2165,44 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     return RT_OK;
 }
 
+// Mirrors the device-side PrepSum (rt_gemm.h).
+struct PrepSum {
+    const float* part;
+    const float* part2;
+    const float* res;
+    float* y;
+    uint32_t splits, crow, full, nch;
+};
+
+// Mirrors the device-side PrepAttn (rt_gemm.h).
+struct PrepAttnHost {
+    const float* part;
+    const float* ml;
+    uint32_t nsp, G, hd, cgs;
+};
+
+// Mirrors the device-side PrepWArgs (k_gemmw.hip).
+struct PrepWArgs {
+    const float* x;
+    const float* gamma;
+    float* xn;
+    void* aops;
+    int* etab;
+    void* ssum;
+    uint32_t M, K;
+    float eps;
+    PrepSum ps;
+    PrepAttnHost pa;
+};
+// The wide form's preparation: mode "", "_n" (RMSNorm), "_sn" (sums, then
+// RMSNorm), "_a" (attention partials).
+static int gemmw_prep(rt_ctx* c, const char* mode, const Gemm3Plan& p, PrepWArgs a) {
+    char pk[48];
+    snprintf(pk, sizeof pk, "k_gemmw_prep%s%s", mode, a.K <= 4096 ? "" : "_l");
+    void* pp[] = {&a};
+    return launch(c, pk, dim3(p.nchunks * 64), dim3(a.K <= 4096 ? 256 : 1024), 0, pp);
+}
+
 // The activation preparation of a plan: x (or RMSNorm(x)·γ with gamma, the
 // normalised rows also into xn when given) into aops / erow / stab.
 static int gemm3_prep(rt_ctx* c, const Gemm3Plan& p, const float* x, uint32_t m_rows, uint32_t k,
@@ -2172,6 +2210,9 @@ static int gemm3_prep(rt_ctx* c, const Gemm3Plan& p, const float* x, uint32_t m_
                       float eps = 0.0f, float* xn = nullptr) {
     const uint32_t MG = p.MG, nchunks = p.nchunks, cu = (uint32_t)c->cu_count;
     uint32_t M = m_rows, K = k;
+    if (MG == 8)
+        return gemmw_prep(c, gamma ? "_n" : "", p,
+                          PrepWArgs{x, gamma, xn, aops, erow, stab, m_rows, k, eps, PrepSum{}, PrepAttnHost{}});
     char pk[48];
     if (gamma) {
         if (k > 20480)
@@ -2868,22 +2909,6 @@ int rt_gemm_qkv_rope_f32(rt_ctx* c, const char* fmt_q, const void* w_q, const ch
                          &rk);
 }
 
-// Mirrors the device-side PrepSum (k_gemm.hip).
-struct PrepSum {
-    const float* part;
-    const float* part2;
-    const float* res;
-    float* y;
-    uint32_t splits, crow, full, nch;
-};
-
-// Mirrors the device-side PrepAttn (k_gemm.hip).
-struct PrepAttnHost {
-    const float* part;
-    const float* ml;
-    uint32_t nsp, G, hd, cgs;
-};
-
 // rt_gemm_ffn_block_f32.  plan_only: report in *shared whether the shared
 // form applies, launching nothing; pa: the O projection's input given as
 // multi-query attention partials (merged in its operand preparation) instead
@@ -2996,10 +3021,15 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         void* aops = at(0);
         int* erow = (int*)at(1);
         float* stab = (float*)at(2);
-        char pk0[48];
-        snprintf(pk0, sizeof pk0, "k_gemm_xh_prep1a_mg%u", po.MG);
-        void* pp0[] = {&pah, &Mr, &Kq, &aops, &erow, &stab};
-        st = launch(c, pk0, dim3(po.nchunks * 8 * po.MG), dim3(1024), 0, pp0);
+        if (MG == 8) {
+            st = gemmw_prep(c, "_a", po, PrepWArgs{nullptr, nullptr, nullptr, aops, erow, stab, Mr, Kq, 0.0f,
+                                                   PrepSum{}, pah});
+        } else {
+            char pk0[48];
+            snprintf(pk0, sizeof pk0, "k_gemm_xh_prep1a_mg%u", po.MG);
+            void* pp0[] = {&pah, &Mr, &Kq, &aops, &erow, &stab};
+            st = launch(c, pk0, dim3(po.nchunks * 8 * po.MG), dim3(1024), 0, pp0);
+        }
     } else {
         st = gemm3_prep(c, po, att, m_rows, qd, at(0), (int*)at(1), (float*)at(2));
     }
@@ -3014,9 +3044,14 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         void* aops = at(3);
         int* erow = (int*)at(4);
         float* stab = (float*)at(5);
-        snprintf(pk, sizeof pk, "k_gemm_xh_prep1sn_mg%u", MG);
-        void* pp[] = {&ps, &M, &K, &aops, &erow, &stab, (void*)&gamma, &eps};
-        st = launch(c, pk, dim3(nch * 8 * MG), dim3(1024), 0, pp);
+        if (MG == 8) {
+            st = gemmw_prep(c, "_sn", po, PrepWArgs{nullptr, gamma, nullptr, aops, erow, stab, M, K, eps, ps,
+                                                    PrepAttnHost{}});
+        } else {
+            snprintf(pk, sizeof pk, "k_gemm_xh_prep1sn_mg%u", MG);
+            void* pp[] = {&ps, &M, &K, &aops, &erow, &stab, (void*)&gamma, &eps};
+            st = launch(c, pk, dim3(nch * 8 * MG), dim3(1024), 0, pp);
+        }
     }
     if (st == RT_OK && MG == 8) {
         // the product silu(gate)·up from the GEMM (the tiles that split K
