@@ -2025,7 +2025,7 @@ static void gemmw_divide(const rt_ctx* c, Gemm3Plan* const* ps, uint32_t count) 
 // Any K that the preparation holds in registers.
 static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                        uint32_t k, Gemm3Plan& p, bool pair = false) {
-    if (m_rows <= c->gemm_wide_min || k > 20480 || !aligned(w, 16) || c->gemm_direct) return false;
+    if (k > 20480 || !aligned(w, 16) || c->gemm_direct) return false;
     p.nblk = k / f.blk_el;
     const bool odd = p.nblk % 2 && !f.has_min;  // rows only 2-byte aligned
     snprintf(p.kn, sizeof p.kn, odd ? "k_gemmw_%s_o" : "k_gemmw_%s", f.name);
@@ -2047,17 +2047,35 @@ static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_ro
     return true;
 }
 
+// Whether a call whose K the staged forms do not tile takes the wide form
+// (the other way: a GEMV a row, for Q8_0 the unstaged GEMM).  Its time hardly
+// depends on the rows below 64; the GEMVs' is theirs times the rows: Q4_0
+// 5000×2080 at 3 / 5 / 32 rows 20 / 34 / 211 against 21 / 20 / 21 µs, 18944×
+// 3616 45 / 73 / 456 against 44 / 41 / 43; Q6_K 3584×18688 at 3 / 4 / 32 57 /
+// 77 / 598 against 52 / 52 / 53, 896×1280 17 / 22 / 177 against 18.  The
+// unstaged GEMM, Q8_0 at 8 / 32 rows: 18944×3616 62 / 80 against 56 / 57 µs,
+// 5000×2080 25 / 31 against 23 / 24, but 896×1056 12 / 14 against 16 / 17.
+static bool gemm_wide_untiled(const rt_ctx* c, const GemmFmt& f, uint32_t m_rows, uint32_t n, uint32_t k) {
+    if (m_rows > c->gemm_wide_min) return true;
+    if (f.blk_bytes == 34) return m_rows > 4 && (uint64_t)n * k >= 1u << 23;
+    return m_rows > (f.blk_bytes == 210 ? 3 : 4);
+}
+
 // Plans the f16 form: 8 activation rows per group (MG ∈ {1, 2, 4}), hi/lo
 // f16 operands prepared by k_gemm_xh_prep*_mg*.  Returns kLsDecline where
 // the staged layout does not apply (the caller then takes the other forms).
-// work: rows × weights of the whole call (0: of this matrix).  The wide form
-// takes calls of gemm_wide_work on, and those whose K the stages here do not tile.
+// work: rows × weights of the whole call (0: of this matrix; UINT64_MAX: the
+// wide form, for a call of which one matrix has no other).  The wide form takes
+// calls above gemm_wide_min rows of gemm_wide_work on, and those whose K the
+// stages here do not tile.
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                       uint32_t k, Gemm3Plan& p, uint64_t work = 0) {
     p = Gemm3Plan{};
     const uint32_t cu = (uint32_t)c->cu_count;
     if (!work) work = (uint64_t)m_rows * n * k;
-    if (work >= c->gemm_wide_work && gemmw_plan(c, f, w, m_rows, n, k, p)) return RT_OK;
+    if ((work == UINT64_MAX || (m_rows > c->gemm_wide_min && work >= c->gemm_wide_work)) &&
+        gemmw_plan(c, f, w, m_rows, n, k, p))
+        return RT_OK;
     const uint32_t groups = (m_rows + 7) / 8;
     const uint32_t MG = std::min<uint32_t>(f.max_mg_f16, groups <= 1 ? 1 : groups <= 2 ? 2 : 4);
     const uint32_t nchunks = (m_rows + 8 * MG - 1) / (8 * MG);
@@ -2078,7 +2096,7 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     }
     const uint32_t seg = NB * f.blk_bytes, vb = seg % 16 == 0 ? 16 : (seg % 8 == 0 ? 8 : 4);
     if (nblk % NB != 0 || !aligned(w, 16) || row_bytes % vb != 0 || c->gemm_direct)
-        return gemmw_plan(c, f, w, m_rows, n, k, p) ? RT_OK : kLsDecline;
+        return gemm_wide_untiled(c, f, m_rows, n, k) && gemmw_plan(c, f, w, m_rows, n, k, p) ? RT_OK : kLsDecline;
     // Q6_K: 128-row tiles with one operand and one weight buffer
     const bool q6 = f.blk_bytes == 210;
     const bool w8ok = !q6 || (c->gemm_q6w8 >> (MG == 4 ? 0 : MG == 2 ? 1 : 2) & 1);

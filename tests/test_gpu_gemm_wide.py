@@ -1,10 +1,11 @@
-"""The wide batched GEMM (k_gemmw_<fmt>, more than 32 activation rows) of every
-block format against the oracle's per-row f64 GEMV of the same packed blocks,
-at the edges of its tiles: rows around one and two 64-row chunks, weight rows
-around 256-row tiles, K of one block, of an odd number of blocks, of one and
-several super-blocks, and K ranges split over workgroups.  Tolerance: every
-output within 1e-4·Σ|w·x| (gpu_helpers); the form's own error is the 22 bits
-of the f16 pairs and some ten f32 roundings, below 1e-6·Σ|w·x|, checked too."""
+"""The wide batched GEMM (k_gemmw_<fmt>, more than 32 activation rows, fewer
+where nothing else tiles K) of every block format against the oracle's per-row
+f64 GEMV of the same packed blocks, at the edges of its tiles: rows around one
+and two 64-row chunks, weight rows around 256-row tiles, K of one block, of an
+odd number of blocks, of one and several super-blocks, and K ranges split over
+workgroups.  Tolerance: every output within 1e-4·Σ|w·x| (gpu_helpers); the
+form's own error is the 22 bits of the f16 pairs and some ten f32 roundings,
+below 1e-6·Σ|w·x|, checked too."""
 import os
 
 import numpy as np
@@ -66,6 +67,30 @@ def test_wide_gemm_block_formats(ctx, fmt, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(33, 3, 256), (64, 257, 768), (129, 300, 4096)])
 def test_wide_gemm_super_block_formats(ctx, fmt, m, n, k):
     _check(ctx, fmt, m, n, k, 920 + m)
+
+
+@pytest.mark.parametrize("fmt,m,n,k", [("q4_0", 5, 70, 32), ("q4_0g", 8, 257, 1056), ("q5_0", 32, 300, 2080),
+                                       ("q8_0", 5, 4096, 2080), ("q8_0", 31, 8200, 1056),
+                                       ("q6k", 4, 257, 256), ("q6kg", 17, 300, 3840), ("q6k", 32, 64, 768)])
+def test_wide_gemm_few_rows(ctx, fmt, m, n, k):
+    """Up to 32 rows, where the staged forms do not tile K."""
+    _check(ctx, fmt, m, n, k, 990 + m)
+
+
+@pytest.mark.parametrize("m", [3, 4, 20])
+def test_wide_set_few_rows_of_mixed_formats(ctx, m):
+    """A set of which only the Q6_K matrix (15 super-blocks a row) has no
+    staged form: below 4 rows separate products, from there on one wide set."""
+    h, n = 3840, 300
+    x = np.random.default_rng(8).standard_normal((m, h)).astype(np.float32)
+    fmts = ["q4k", "q4k", "q6k"]
+    W = [device_weights(ctx, f, n, h, 995 + i) for i, f in enumerate(fmts)]
+    ys = [ctx.new_buffer(4 * m * n) for _ in fmts]
+    d.gemm_set_f32(ctx, fmts, [w for w, _ in W], ys, [n] * 3, ctx.buffer_from(x), m, h)
+    ctx.flush()
+    for f, y, (_, raw) in zip(fmts, ys, W):
+        ref, sabs = ora.gemv(f, raw, x, n, h)
+        check_close(y.read(np.float32, m * n), ref.ravel(), sabs.ravel(), f"{f} of a mixed set of {m} rows")
 
 
 @pytest.mark.parametrize("fmt", ["q8_0", "q4kg"])
