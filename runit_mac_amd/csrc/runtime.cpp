@@ -139,6 +139,8 @@ const char* const kKernelNames[] = {
     "k_rms_norm_f32g", "k_rope_qk_f32", "k_kv_copy_f32",
     "k_decode_attention_f32_hd64", "k_decode_attention_f32_hd128", "k_decode_attention_f32_hd256",
     "k_attn_mq_f32_hd64", "k_attn_mq_f32_hd128", "k_attn_mq_f32_hd256",
+    "k_attn_pf_prep_hd64", "k_attn_pf_prep_hd128", "k_attn_pf_f32_hd64", "k_attn_pf_f32_hd128",
+    "k_attn_pf_merge_hd64", "k_attn_pf_merge_hd128",
     "k_attn_rope_f32_hd64", "k_attn_rope_f32_hd128", "k_attn_rope_f32_hd256",
     "k_attn_rope_w_f32_hd64", "k_attn_rope_w_f32_hd128",
     "k_add_f16_into_f32", "k_ssq_quads", "k_add_bias_broadcast_f32", "k_rope_batch_f32", "k_kv_write_batch_f32",
@@ -315,6 +317,10 @@ struct rt_ctx {
     uint32_t gemm_splits = 0;    // RUNIT_GEMM_SPLITS=n: the f16 GEMM's K splits forced (A/B)
     bool attn_w = true;          // RUNIT_ATTN_W=0: the token's RoPE attention on attn_split (A/B)
     bool attn_mq = true;         // RUNIT_ATTN_MQ=0: multi-query attention on attn_split per row (A/B)
+    // RUNIT_ATTN_PF_WORK: query heads × positions from which a prompt's attention takes the f16
+    // form (0: every one it can; tests, A/B); RUNIT_ATTN_PF_NSP: its ranges (0: planned)
+    uint64_t attn_pf_work = 3000000;
+    uint32_t attn_pf_nsp = 0;
     uint32_t attn_mq_nsp = 0, attn_mq_w = 0;  // probe: forced ranges / waves (0: planned)
     // RUNIT_ATTN_MQ_MIN / _FOLD_MIN: column-group pairs up to which the
     // per-row kernel runs (rt_flash_attention_f32 / rt_gemm_attn_ffn_block_f32)
@@ -1363,6 +1369,8 @@ int rt_ctx_create(rt_ctx** out, const char* code_object_path) {
     if (const char* g = getenv("RUNIT_GEMM_F16_MIN_Q6")) c->gemm_f16_min_q6 = (uint32_t)atoi(g);
     if (const char* g = getenv("RUNIT_ATTN_W")) c->attn_w = atoi(g) != 0;
     if (const char* g = getenv("RUNIT_ATTN_MQ")) c->attn_mq = atoi(g) != 0;
+    if (const char* g = getenv("RUNIT_ATTN_PF_WORK")) c->attn_pf_work = strtoull(g, nullptr, 10);
+    if (const char* g = getenv("RUNIT_ATTN_PF_NSP")) c->attn_pf_nsp = atoi(g);
     if (const char* g = getenv("RUNIT_ATTN_MQ_NSP")) c->attn_mq_nsp = atoi(g);
     if (const char* g = getenv("RUNIT_ATTN_MQ_MIN")) c->attn_mq_min = atoi(g);
     if (const char* g = getenv("RUNIT_ATTN_MQ_FOLD_MIN")) c->attn_mq_fold_min = atoi(g);
@@ -3851,6 +3859,73 @@ static int attn_mq_launch(rt_ctx* c, AttnArgs a, uint32_t batch, uint32_t q_len,
     return kLsDecline;
 }
 
+// Mirrors the device-side AttnPfArgs (k_attn.hip).
+struct AttnPfArgs {
+    const float* q;
+    const float* kc;
+    const float* vc;
+    float* out;
+    void* ops;
+    float* part;
+    float* ml;
+    uint32_t kv, stride, H, KVH, q_len, q_start, tiles, cbs, nsp, items;
+    float scale;
+};
+
+// The attention of long prompts (k_attn_pf_*): keys and values prepared, the
+// products on the f16 matrix cores, the ranges merged.  kLsDecline where
+// k_attn_mq is the better one, or the workspace cannot hold it.
+static int attn_pf_launch(rt_ctx* c, const AttnArgs& a, uint32_t batch, uint32_t head_dim) {
+    if (!c->attn_mq || (head_dim != 64 && head_dim != 128) || batch > 65535) return kLsDecline;
+    const uint32_t kv = std::min<uint64_t>(a.kv_len, (uint64_t)a.q_start + a.q_len);
+    const uint64_t rows = (uint64_t)batch * a.q_len * a.H, cols = (uint64_t)a.q_len * (a.H / a.KVH);
+    // From 1,024 positions on: fewer are too little work for its three launches
+    // (28 heads of 128, 128 queries: 20 against 11 µs; 256: 28 / 27), and the
+    // f16 pairs' own error, which does not grow with the positions, exceeds the
+    // f32 form's there (300 queries: 1.6e-7 against 1.3e-7; after 500
+    // positions level at 2.2e-7; after 1,000 2.5e-7 against 2.8e-7; 512 after
+    // 1,536 3.4e-7 against 4.3e-7).  And from 3e6 scores on: 64 queries after
+    // 1,000 (1.9e6) 29 against 28 µs, 128 after 1,000 (4.0e6) 33 / 38, 64 after
+    // 4,000 (7.3e6) 53 / 67, 512 after 1,536 (29e6) 79 / 182, 2,048 alone 155 /
+    // 482; 14 heads of 64, 300 after 1,000 (5.5e6) 27 / 40.
+    if (c->attn_pf_work && (kv < 1024 || rows * kv < c->attn_pf_work)) return kLsDecline;
+    // ranges of the positions for about two workgroups on every CU, each of at
+    // least 4 records of 32; twice as many where the first query sees less than
+    // half of what the last one does, as the workgroups then differ in length
+    // (28 heads of 128, 512 queries after 1,536: 2 / 4 / 8 ranges 100 / 83 /
+    // 93 µs; 2,048 queries alone: 1 / 2 / 6 ranges 181 / 163 / 205)
+    const uint32_t tiles = (kv + 31) / 32, cbs = (uint32_t)((cols + 127) / 128);
+    const uint64_t wgs = (uint64_t)cbs * a.KVH * batch;
+    const uint64_t slots = (a.q_start < kv / 2 ? 4ull : 2ull) * c->cu_count;
+    uint32_t nsp = std::max<uint64_t>(1, std::min<uint64_t>({slots / wgs, tiles / 4, RT_ATTN_MQ_NSP_MAX}));
+    if (c->attn_pf_nsp) nsp = std::min({c->attn_pf_nsp, tiles, RT_ATTN_MQ_NSP_MAX});
+    if (wgs * nsp > 0x7FFFFF00ull) return kLsDecline;
+    const size_t o_bytes = (size_t)batch * a.KVH * tiles * (head_dim * 16 + 64) * 16;
+    const size_t parts = nsp > 1 ? (size_t)wgs * nsp * 128 : 0;
+    const size_t bytes = o_bytes + parts * (head_dim + 2) * sizeof(float);
+    if (bytes > c->ws_bytes) {
+        if (c->capturing || c->noalloc) return kLsDecline;
+        // for the whole cache, so that the growing prefixes of a prompt in
+        // chunks find it sized (outgrown workspaces stay until the context ends)
+        const size_t all = (size_t)batch * a.KVH * ((a.stride + 31) / 32) * (head_dim * 16 + 64) * 16 +
+                           (wgs <= 2ull * c->cu_count ? 4ull * c->cu_count * 128 * (head_dim + 2) * sizeof(float) : 0);
+        if (ensure_ws(c, std::max(bytes, all), "flash_attention") != RT_OK) return kLsDecline;
+    }
+    float* part = parts ? (float*)((char*)c->ws + o_bytes) : nullptr;
+    AttnPfArgs p{a.q, a.kc, a.vc, a.out, c->ws, part, part ? part + parts * head_dim : nullptr, kv, a.stride, a.H,
+                 a.KVH, a.q_len, a.q_start, tiles, cbs, nsp, (uint32_t)(wgs * nsp), a.scale};
+    void* params[] = {&p};
+    char kn[48];
+    snprintf(kn, sizeof kn, "k_attn_pf_prep_hd%u", head_dim);
+    int st = launch(c, kn, dim3(tiles, a.KVH, batch), dim3(2 * head_dim), 0, params);
+    if (st != RT_OK) return st;
+    snprintf(kn, sizeof kn, "k_attn_pf_f32_hd%u", head_dim);
+    st = launch(c, kn, dim3((p.items + 7) / 8 * 8), dim3(256), 0, params);
+    if (st != RT_OK || nsp == 1) return st;
+    snprintf(kn, sizeof kn, "k_attn_pf_merge_hd%u", head_dim);
+    return launch(c, kn, dim3((uint32_t)((cols * (head_dim / 4) + 255) / 256), a.KVH, batch), dim3(256), 0, params);
+}
+
 int rt_gemm_attn_ffn_block_f32(rt_ctx* c, const float* q, const float* k_cache,
                                const float* v_cache, uint32_t kv_len, uint32_t num_heads,
                                uint32_t num_kv_heads, uint32_t head_dim, uint32_t kv_head_stride,
@@ -3935,6 +4010,8 @@ int rt_flash_attention_f32(rt_ctx* c, const float* q, const float* k, const floa
     a.q_len = q_len;
     a.q_start = q_start;
     char kn[64];
+    st = attn_pf_launch(c, a, batch, head_dim);
+    if (st != kLsDecline) return st;
     const int mq = attn_mq_launch(c, a, batch, q_len, kv_len, num_heads, num_kv_heads, head_dim,
                                   q_start, c->attn_mq_min, false, false, nullptr);
     if (mq != kLsDecline) return mq;

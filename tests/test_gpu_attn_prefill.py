@@ -1,0 +1,119 @@
+"""The long-prompt attention (k_attn_pf_f32_hd64 / 128) against the oracle's
+causal attention: the edges of its 128-column workgroups and 32-position
+records, positions split over workgroups, sequences of a batch, keys and
+values of magnitudes far apart, infinities.  Tolerance: a convex combination
+of values with an f32 softmax, 1e-5 of the value range (test_gpu_verify)."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle_lib as ora
+from runit_mac_amd import dispatch as d
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    """A context whose attention takes this form however short the prompt."""
+    os.environ["RUNIT_ATTN_PF_WORK"] = "0"
+    try:
+        c = d.HipContext()
+    finally:
+        del os.environ["RUNIT_ATTN_PF_WORK"]
+    yield c
+    c.close()
+
+
+def run(ctx, q, kc, vc, batch, M, kv_len, H, KVH, hd, S, q_start):
+    bo = ctx.new_buffer(4 * (batch * M * H * hd + 64))
+    bo.write(np.full(batch * M * H * hd + 64, 7.0, np.float32))
+    d.flash_attention_f32(ctx, ctx.buffer_from(q), ctx.buffer_from(kc), ctx.buffer_from(vc), bo, batch, M, kv_len, H,
+                          KVH, hd, S, q_start)
+    assert d.last_launch_name(ctx) in (f"k_attn_pf_f32_hd{hd}", f"k_attn_pf_merge_hd{hd}")
+    ctx.flush()
+    got = bo.read(np.float32, batch * M * H * hd + 64)
+    assert np.all(got[batch * M * H * hd:] == 7.0), "past the last row"
+    return got[:batch * M * H * hd].reshape(batch, M, H * hd)
+
+
+@pytest.mark.parametrize("hd,H,KVH,M,kv_len,q_start", [
+    (64, 1, 1, 1, 1, 0),          # one query, one position
+    (128, 2, 2, 33, 33, 0),       # one column block, the second record of one position
+    (64, 14, 2, 19, 200, 181),    # 133 columns: a second block of 5
+    (128, 28, 4, 40, 300, 260),   # position ranges merged
+    (64, 8, 8, 130, 130, 0),      # ranges that the first block does not see
+    (128, 6, 2, 50, 64, 30),      # rows past kv_len: all of it
+    (64, 4, 2, 300, 1000, 700),
+])
+def test_prefill_attention(ctx, hd, H, KVH, M, kv_len, q_start):
+    rng = np.random.default_rng(hd + M + kv_len)
+    S = kv_len + 16
+    q = rng.standard_normal(M * H * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal(KVH * S * hd).astype(np.float32) for _ in range(2))
+    # past the last position that a query sees the cache is not read
+    last = min(kv_len, q_start + M)
+    for x in (kc, vc):
+        x.reshape(KVH, S, hd)[:, last:] = np.nan
+    got = run(ctx, q, kc, vc, 1, M, kv_len, H, KVH, hd, S, q_start)[0]
+    ref = ora.causal_attention(q, kc, vc, M, H, KVH, hd, kv_len, S, q_start)
+    assert np.max(np.abs(got - ref)) <= 1e-5 * np.nanmax(np.abs(vc))
+
+
+def test_prefill_attention_batch(ctx):
+    rng = np.random.default_rng(9)
+    hd, H, KVH, M, kv_len, S = 64, 6, 2, 50, 300, 310
+    q = rng.standard_normal(2 * M * H * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal(2 * KVH * S * hd).astype(np.float32) for _ in range(2))
+    got = run(ctx, q, kc, vc, 2, M, kv_len, H, KVH, hd, S, kv_len - M)
+    per = KVH * S * hd
+    for b in range(2):
+        ref = ora.causal_attention(q.reshape(2, -1)[b], kc[b * per:(b + 1) * per], vc[b * per:(b + 1) * per], M, H,
+                                   KVH, hd, kv_len, S, kv_len - M)
+        assert np.max(np.abs(got[b] - ref)) <= 1e-5 * np.abs(vc).max(), b
+
+
+def test_prefill_attention_scales(ctx):
+    """Keys, queries and values whose magnitudes differ by 2^40 from row to
+    row (scores of every size, exponents of records rising and falling), and
+    all-zero rows: the error of each output within 1e-5 of the values its
+    query weights, Σ p·|v|."""
+    rng = np.random.default_rng(11)
+    hd, H, KVH, M, S = 128, 2, 1, 70, 200
+    q = rng.standard_normal((M, H, hd)).astype(np.float32)
+    kc = rng.standard_normal((S, hd)).astype(np.float32)
+    vc = rng.standard_normal((S, hd)).astype(np.float32)
+    q *= np.exp2(rng.integers(-20, 1, (M, 1, 1))).astype(np.float32)
+    kc *= np.exp2(rng.integers(-20, 1, (S, 1))).astype(np.float32)
+    vc *= np.exp2(rng.integers(-20, 21, S // 8).repeat(8)[:, None]).astype(np.float32)
+    vc[40:80] *= 2.0 ** -60
+    q[3], kc[5], vc[64:96] = 0, 0, 0
+    got = run(ctx, q.ravel(), kc.ravel(), vc.ravel(), 1, M, S, H, KVH, hd, S, S - M)[0]
+    ref = ora.causal_attention(q.ravel(), kc.ravel(), vc.ravel(), M, H, KVH, hd, S, S, S - M)
+    mag = ora.causal_attention(q.ravel(), kc.ravel(), np.abs(vc).ravel(), M, H, KVH, hd, S, S, S - M)
+    assert np.all(np.abs(got - ref) <= 1e-5 * mag)
+
+
+def test_prefill_attention_infinities(ctx):
+    """A key of -inf score leaves its position out, one of +inf makes the rows
+    that see it NaN, an infinite value its element infinite: as in f32
+    throughout; rows that do not see them are untouched."""
+    rng = np.random.default_rng(12)
+    hd, H, KVH, M, S = 64, 2, 1, 90, 100
+    q = np.abs(rng.standard_normal((M, H, hd))).astype(np.float32)
+    kc, vc = (rng.standard_normal((S, hd)).astype(np.float32) for _ in range(2))
+    clean = (q.ravel(), kc.copy(), vc.copy())
+    kc[20, 7] = -np.inf
+    kc[70, 3] = np.inf
+    vc[45, 9] = np.inf
+    got = run(ctx, q.ravel(), kc.ravel(), vc.ravel(), 1, M, M, H, KVH, hd, S, 0)[0].reshape(M, H, hd)
+    low = clean[1].copy()
+    low[20] = -1e4 * np.ones(hd)  # (a score below every other by far)
+    for lo, hi, keys in ((0, 20, clean[1]), (20, 70, low)):
+        ref = ora.causal_attention(clean[0], keys.ravel(), clean[2].ravel(), M, H, KVH, hd, M, S, 0).reshape(M, H, hd)
+        for r in range(lo, hi):
+            e = np.arange(hd) != 9 if r >= 32 else np.ones(hd, bool)  # (0·inf in the record of value 45 is NaN)
+            assert np.max(np.abs(got[r][:, e] - ref[r][:, e])) <= 1e-5 * np.abs(clean[2]).max(), r
+    assert np.all(np.isinf(got[45:70, :, 9]))
+    assert np.all(np.isnan(got[70:]))
