@@ -516,6 +516,9 @@ int ensure_ws(rt_ctx* c, size_t need, const char* who) {
 int ensure_part(rt_ctx* c, size_t need, const char* who) {
     return ensure_buf(c, c->part, c->part_bytes, need, who);
 }
+// Whether the workspace holds `need` bytes or may grow to: a form that needs
+// more than its predecessor on a shape leaves the call to it where not.
+bool ws_holds(const rt_ctx* c, size_t need) { return need <= c->ws_bytes || !(c->capturing || c->noalloc); }
 
 bool has_ls_kernel(const rt_ctx* c, const char* kname) {
     return c->fns.count(std::string(kname) + "_ls1") != 0;
@@ -2104,7 +2107,10 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     }
     const uint32_t seg = NB * f.blk_bytes, vb = seg % 16 == 0 ? 16 : (seg % 8 == 0 ? 8 : 4);
     if (nblk % NB != 0 || !aligned(w, 16) || row_bytes % vb != 0 || c->gemm_direct)
-        return gemm_wide_untiled(c, f, m_rows, n, k) && gemmw_plan(c, f, w, m_rows, n, k, p) ? RT_OK : kLsDecline;
+        return gemm_wide_untiled(c, f, m_rows, n, k) && gemmw_plan(c, f, w, m_rows, n, k, p) &&
+                       ws_holds(c, p.a_bytes + p.e_bytes + p.s_bytes + p.p_bytes)
+                   ? RT_OK
+                   : kLsDecline;
     // Q6_K: 128-row tiles with one operand and one weight buffer
     const bool q6 = f.blk_bytes == 210;
     const bool w8ok = !q6 || (c->gemm_q6w8 >> (MG == 4 ? 0 : MG == 2 ? 1 : 2) & 1);
@@ -2688,6 +2694,7 @@ static int gemm_set_wide(rt_ctx* c, uint32_t count, const GemmFmt* const* f, Gem
         psize[i] = (psize[i] + 255) & ~(size_t)255;
         total += pair ? 2 * psize[i] : psize[i];
     }
+    if (!ws_holds(c, total)) return kLsDecline;
     int st = ensure_ws(c, total, "gemm_set");
     if (st != RT_OK) return st;
     char* ws = (char*)c->ws;
@@ -2797,6 +2804,12 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
         if (st != RT_OK && st != kLsDecline) return st;
         shared = st == RT_OK && pl[i].MG == pl[0].MG;
     }
+    if (shared && pl[0].MG == 8) {
+        const int st = gemm_set_wide(c, count, f, pl, w, y, n, bias, res, x, m_rows, k, gamma, eps, xn,
+                                     silu_pair, rope);
+        if (st != kLsDecline) return st;
+        shared = false;
+    }
     if (!shared) {
         // the separate launches: norm, one GEMM per matrix, then the
         // bias / residual / SiLU kernels
@@ -2820,9 +2833,6 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
                                               m_rows, rope->max_seq);
         return RT_OK;
     }
-    if (pl[0].MG == 8)
-        return gemm_set_wide(c, count, f, pl, w, y, n, bias, res, x, m_rows, k, gamma, eps, xn,
-                             silu_pair, rope);
     // workspace: [operands | row exponents | record sums | partials of each matrix]
     bool any_min = false;
     for (uint32_t i = 0; i < count; ++i) any_min |= f[i]->has_min;
@@ -3000,10 +3010,6 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
                          (po.MG == 8 ? fg != fu : pg.splits != pu.splits))))
         return plan_only ? RT_OK : sets();
     if (st != RT_OK) return st;
-    if (plan_only) {
-        if (shared) *shared = true;
-        return RT_OK;
-    }
     // workspace: operands of att (K = qd), of the normalised x_mid (K = h),
     // of the SiLU product (K = ff), then the partial sums of O, gate, up, down
     const uint32_t MG = po.MG, nch = po.nchunks, crow = 8 * MG;
@@ -3031,6 +3037,11 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     }
     const size_t off_pd = total;
     total += parts(pd, h);
+    if (MG == 8 && !ws_holds(c, total)) return plan_only ? RT_OK : sets();
+    if (plan_only) {
+        if (shared) *shared = true;
+        return RT_OK;
+    }
     st = ensure_ws(c, total, "gemm_ffn_block");
     if (st != RT_OK) return st;
     char* ws = (char*)c->ws;
@@ -3903,8 +3914,8 @@ static int attn_pf_launch(rt_ctx* c, const AttnArgs& a, uint32_t batch, uint32_t
     const size_t o_bytes = (size_t)batch * a.KVH * tiles * (head_dim * 16 + 64) * 16;
     const size_t parts = nsp > 1 ? (size_t)wgs * nsp * 128 : 0;
     const size_t bytes = o_bytes + parts * (head_dim + 2) * sizeof(float);
+    if (!ws_holds(c, bytes)) return kLsDecline;
     if (bytes > c->ws_bytes) {
-        if (c->capturing || c->noalloc) return kLsDecline;
         // for the whole cache, so that the growing prefixes of a prompt in
         // chunks find it sized (outgrown workspaces stay until the context ends)
         const size_t all = (size_t)batch * a.KVH * ((a.stride + 31) / 32) * (head_dim * 16 + 64) * 16 +

@@ -117,3 +117,37 @@ def test_prefill_attention_infinities(ctx):
             assert np.max(np.abs(got[r][:, e] - ref[r][:, e])) <= 1e-5 * np.abs(clean[2]).max(), r
     assert np.all(np.isinf(got[45:70, :, 9]))
     assert np.all(np.isnan(got[70:]))
+
+
+def test_prefill_attention_capture():
+    """Captured in a context whose workspace is not sized the call keeps the
+    kernel that needs none; after an eager call it is captured in this form,
+    and replays after eager work of its own give the eager result."""
+    hd, H, KVH, M, S = 64, 14, 2, 300, 300
+    rng = np.random.default_rng(13)
+    q = rng.standard_normal(M * H * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal(KVH * S * hd).astype(np.float32) for _ in range(2))
+    os.environ["RUNIT_ATTN_PF_WORK"] = "0"
+    try:
+        ctx = d.HipContext()
+    finally:
+        del os.environ["RUNIT_ATTN_PF_WORK"]
+    with ctx:
+        bufs = [ctx.buffer_from(a) for a in (q, kc, vc)]
+        bo = ctx.new_buffer(4 * M * H * hd)
+        call = lambda: d.flash_attention_f32(ctx, *bufs, bo, 1, M, S, H, KVH, hd, S, 0)
+        ref = ora.causal_attention(q, kc, vc, M, H, KVH, hd, S, S, 0)
+        for kernel in (f"k_attn_mq_f32_hd{hd}", f"k_attn_pf_merge_hd{hd}"):
+            ctx.capture_begin()
+            call()
+            g = ctx.capture_end()
+            assert d.last_launch_name(ctx) == kernel
+            for _ in range(3):
+                bo.write(np.zeros(M * H * hd, np.float32))
+                g.launch()
+                ctx.flush()
+                got = bo.read(np.float32, M * H * hd).reshape(M, H * hd)
+                assert np.max(np.abs(got - ref)) <= 1e-5 * np.abs(vc).max()
+                call()  # (eager; sizes the workspace the first time)
+                ctx.flush()
+            del g

@@ -165,3 +165,31 @@ def test_wide_qkv_rope_equals_set_then_rope(ctx):
     for a, b, what in zip(outs[0][:2], outs[1][:2], ("q", "k cache")):
         assert np.max(np.abs(a - b)) <= 2e-6 * np.abs(b).max(), what
     assert np.array_equal(outs[0][2], outs[1][2]), "v cache"
+
+
+def test_wide_gemm_few_rows_capture():
+    """In a context without a workspace, a captured call (and set) of a K that
+    nothing tiles runs a GEMV a row as before this form; after an eager call,
+    this form; every replay gives the result."""
+    m, n, k = 8, 300, 1056
+    x = np.random.default_rng(14).standard_normal((m, k)).astype(np.float32)
+    with d.HipContext() as ctx:
+        W = [device_weights(ctx, "q4_0", n, k, 1010 + i) for i in range(2)]
+        xb, ys = ctx.buffer_from(x), [ctx.new_buffer(4 * m * n) for _ in range(2)]
+        refs = [ora.gemv("q4_0", raw, x, n, k) for _, raw in W]
+        for call, outs in ((lambda: d.gemm_q4_0_f32(ctx, W[0][0], xb, ys[0], m, n, k), 1),
+                           (lambda: d.gemm_set_f32(ctx, ["q4_0"] * 2, [w for w, _ in W], ys, [n, n], xb, m, k), 2)):
+            for _ in range(2):
+                ctx.capture_begin()
+                call()
+                g = ctx.capture_end()
+                for _ in range(2):
+                    for y in ys:
+                        y.write(np.zeros(m * n, np.float32))
+                    g.launch()
+                    ctx.flush()
+                    for y, (ref, sabs) in list(zip(ys, refs))[:outs]:
+                        check_close(y.read(np.float32, m * n), ref.ravel(), sabs.ravel(), "captured")
+                    call()
+                    ctx.flush()
+                del g
