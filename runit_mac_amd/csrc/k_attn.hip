@@ -1,19 +1,21 @@
 // k_attn.hip — causal multi-query attention of long prompts: keys and values
-// prepared once a call as pairs of f16 (x·2^e = hi + lo, 22 bits and more), both
-// products on the 32x32x16 f16 matrix cores (f16 × f16 products exact, f32
-// sums), the softmax in f32.
+// prepared once a call as pairs of f16 (x·2^e = hi + lo, an exponent a row: 22
+// bits of the elements down to 2^-18 of the row's largest, 2^-40 of that
+// below), both products on the 32x32x16 f16 matrix cores (f16 × f16 products
+// exact, f32 sums), the softmax in f32.
 //
 // k_attn_mq's f32 matrix cores bound it, a sixteenth of the f16 rate, and its
 // operand loads, 64 lines of L1 an instruction: 512 queries of 28 heads of 128
 // after 1,536 positions ran 182 µs, 13 GFLOP at 72 of 157 TFLOP/s.  Three f16
 // products (hi·hi, hi·lo, lo·hi) take 3/16 of the f32 product's matrix time:
-// 79 µs here, of which the preparation is 6, the merge of the ranges 8 and
-// about 15 the start and end of the main kernel's workgroups.  A record then
-// costs 1.6 µs with one workgroup on a CU and 2.6 with two: 0.65 of it are the
-// matrix cores, each wave's softmax hides behind them only in part.
-// Measured on the way: expf instead of exp2 (VALU 780 instead of 350
-// instructions a record) 95 µs, the operands loaded where they are used 82,
-// the sums rescaled at each new maximum 80.
+// 81 µs here, of which the preparation is 8, the merge of the ranges 8 and
+// about 15 the start and end of the main kernel's workgroups: 0.65 µs a record
+// and wave are the matrix cores, each wave's softmax hides behind them only in
+// part.  (One exponent for all values of a record, put into P before it is
+// split, ran 75: it lost the weights of values far below the largest that any
+// record held.)  Measured on the way, from 79 µs: expf instead of exp2 95, the
+// operands loaded where they are used 82, the sums rescaled at each new
+// maximum 80.
 #include "rt_attn.h"
 
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -37,11 +39,16 @@ struct AttnPfArgs {
 };
 
 // A record: the key operands [HD/16 steps][hi, lo][64 lanes], the value
-// operands [HD/32 blocks][2 steps][hi, lo][64], then 256 words: 2^-exponent of
-// the 32 keys, the exponent of the values, whether a key or value is not finite.
+// operands [HD/32 blocks][2 steps][hi, lo][64], then 256 words (PfTail on).
 template <int HD>
 struct PfRec {
     static constexpr uint32_t OPS = HD * 16, LEN = OPS + 64;  // in 16-byte entries
+};
+enum PfTail {
+    kTailK = 0,    // 2^-exponent of the 32 keys
+    kTailV = 32,   // of the 32 values, 0 of an all-zero one
+    kTailMax = 64, // exponent of the largest value (int)
+    kTailBad = 65, // whether a key or value is not finite (int)
 };
 
 // x·f as hi + lo
@@ -60,8 +67,9 @@ RT_DEV int pf_exp(float mx) { return mx > 0.0f ? min(126, 15 - __builtin_amdgcn_
 RT_DEV float pf_pow2(int e) { return ldexpf(1.0f, e); }
 
 // One workgroup a record (2·HD threads): every position of the cache is read
-// once and written in as many bytes, in the order that the operands of
-// attn_pf take them.  Keys: lane l of step s holds d = 16s + 8(l / 32) .. of
+// once (its value a second time, from L2) and written in as many bytes, in the
+// order that the operands of attn_pf take them, each key and each value scaled
+// by an exponent of its own.  Keys: lane l of step s holds d = 16s + 8(l / 32) .. of
 // position l % 32.  Values: lane l of (block b, step s) holds d = 32b + l % 32
 // at the positions whose scores its half of the wave has in registers 8s ..
 // 8s + 7 of the score tile: 16s + 8(i / 4) + 4(l / 32) + i % 4.
@@ -69,6 +77,7 @@ template <int HD>
 RT_DEV void attn_pf_prep(const AttnPfArgs& a) {
     constexpr uint32_t KS = HD / 16;
     __shared__ float red[16];
+    __shared__ float vscale[32];
     const uint32_t t = blockIdx.x, tid = threadIdx.x;
     const size_t seq = (size_t)blockIdx.z * a.KVH + blockIdx.y;
     const float* kb = a.kc + seq * a.stride * HD;
@@ -77,33 +86,35 @@ RT_DEV void attn_pf_prep(const AttnPfArgs& a) {
     float* tail = (float*)(rec + PfRec<HD>::OPS);
     bool bad = false;
     const uint32_t p = tid / KS, s = tid % KS;
-    float x[2][8] = {}, v[2][8];
+    float x[2][8] = {}, vmax = 0.0f, kmax = 0.0f;
     if (t * 32 + p < a.kv) {
         const f32x4* k4 = (const f32x4*)(kb + (size_t)(t * 32 + p) * HD + 16 * s);
+        const f32x4* v4 = (const f32x4*)(vb + (size_t)(t * 32 + p) * HD + 16 * s);
 #pragma unroll
-        for (uint32_t i = 0; i < 16; ++i) x[i / 8][i % 8] = k4[i / 4][i % 4];
-    }
-    float vmax = 0.0f, kmax = 0.0f;
-#pragma unroll
-    for (uint32_t r = 0; r < 2; ++r) {
-        const uint32_t idx = tid + 2 * HD * r, l = idx & 63, bs = idx >> 6;
-        const uint32_t d = 32 * (bs / 2) + (l & 31);
-#pragma unroll
-        for (uint32_t i = 0; i < 8; ++i) {
-            const uint32_t pos = t * 32 + 16 * (bs % 2) + 8 * (i / 4) + 4 * (l >> 5) + i % 4;
-            v[r][i] = pos < a.kv ? vb[(size_t)pos * HD + d] : 0.0f;
+        for (uint32_t i = 0; i < 16; ++i) {
+            x[i / 8][i % 8] = k4[i / 4][i % 4];
+            const float av = fabsf(v4[i / 4][i % 4]), ak = fabsf(x[i / 8][i % 8]);
+            bad |= !(av < __builtin_huge_valf()) || !(ak < __builtin_huge_valf());
+            vmax = fmaxf(vmax, av);
+            kmax = fmaxf(kmax, ak);
         }
     }
-#pragma unroll
-    for (uint32_t i = 0; i < 16; ++i) {
-        const float av = fabsf(v[i / 8][i % 8]), ak = fabsf(x[i / 8][i % 8]);
-        bad |= !(av < __builtin_huge_valf()) || !(ak < __builtin_huge_valf());
-        vmax = fmaxf(vmax, av);
-        kmax = fmaxf(kmax, ak);
+    for (uint32_t o = 1; o < KS; o *= 2) {
+        kmax = fmaxf(kmax, __shfl_xor(kmax, o, 64));
+        vmax = fmaxf(vmax, __shfl_xor(vmax, o, 64));
     }
-    for (uint32_t o = 1; o < KS; o *= 2) kmax = fmaxf(kmax, __shfl_xor(kmax, o, 64));
-    const int ke = pf_exp(kmax), ve = pf_exp(block_max(vmax, red));
+    const int ke = pf_exp(kmax), ve = pf_exp(vmax);
+    if (s == 0) {
+        vscale[p] = pf_pow2(ve);
+        tail[kTailK + p] = pf_pow2(-ke);
+        tail[kTailV + p] = vmax > 0.0f ? pf_pow2(-ve) : 0.0f;
+    }
+    const int vexp = pf_exp(block_max(vmax, red));  // (also the barrier before vscale is read)
     const float any = block_max(bad ? 1.0f : 0.0f, red);
+    if (tid == 0) {
+        ((int*)tail)[kTailMax] = vexp;
+        ((int*)tail)[kTailBad] = any != 0.0f;
+    }
     h8_t hi, lo;
 #pragma unroll
     for (uint32_t h = 0; h < 2; ++h) {
@@ -114,14 +125,16 @@ RT_DEV void attn_pf_prep(const AttnPfArgs& a) {
 #pragma unroll
     for (uint32_t r = 0; r < 2; ++r) {
         const uint32_t idx = tid + 2 * HD * r, l = idx & 63, bs = idx >> 6;
-        pf_split(v[r], pf_pow2(ve), hi, lo);
+        const uint32_t d = 32 * (bs / 2) + (l & 31);
+        float v[8];
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i) {
+            const uint32_t pos = 16 * (bs % 2) + 8 * (i / 4) + 4 * (l >> 5) + i % 4;
+            v[i] = t * 32 + pos < a.kv ? vb[(size_t)(t * 32 + pos) * HD + d] * vscale[pos] : 0.0f;
+        }
+        pf_split(v, 1.0f, hi, lo);
         rec[PfRec<HD>::OPS / 2 + 2 * bs * 64 + l] = hi;
         rec[PfRec<HD>::OPS / 2 + (2 * bs + 1) * 64 + l] = lo;
-    }
-    if (s == 0) tail[p] = pf_pow2(-ke);
-    if (tid == 0) {
-        ((int*)tail)[32] = ve;
-        ((int*)tail)[33] = any != 0.0f;
     }
 }
 
@@ -130,10 +143,13 @@ RT_DEV void attn_pf_prep(const AttnPfArgs& a) {
 // see; wave w takes columns 32w ...  The next record goes to LDS while this
 // one is computed (33 KB each at head size 128: two workgroups a CU).  Per
 // record a wave computes Sᵀ = K·Qᵀ (a lane: 16 of the 32 positions of one
-// column), the online softmax, and Oᵀ += Vᵀ·Pᵀ with P·2^6 split as the rest.
-// The values' exponents differ between records: the sums stand at the
-// smallest so far, and P is scaled down where a record's is above it.  A
-// record that holds an infinity or NaN is computed in plain f32, from the cache.
+// column), the online softmax, and Oᵀ += Vᵀ·Pᵀ.  P is split as the rest after
+// the values' scales were put into it: each weight is then as large as what
+// its position contributes, the column's largest in [2^14, 2^15), so that a
+// value's rounding is measured by its own part of the output, whatever the
+// magnitudes of the others, of unseen ones or of ones whose weight is nothing.
+// The record's product starts at zero and is added in f32.  A record that holds an
+// infinity or NaN is computed in plain f32, from the cache.
 template <int HD>
 RT_DEV void attn_pf(const AttnPfArgs& a) {
     constexpr uint32_t PF = 3;  // operands loaded two steps ahead
@@ -191,7 +207,6 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
     // a column's reference, near its largest score so far, in units of log 2,
     // and what is taken off its scores (0 while nothing is seen)
     float m = NEG, md = 0.0f, l = 0.0f;
-    int eref = 1000;
     const float scale2 = a.scale * 1.44269504f, qf = scale2 * pf_pow2(-eq);
     for (uint32_t t = t0; t < t1; ++t) {
         const uint32_t buf = (t - t0) & 1, p0 = t * 32;
@@ -206,8 +221,9 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
         if (p0 < Lw) {
             const h8_t* op = (const h8_t*)lds[buf] + lane;
             const float* tail = (const float*)&lds[buf][OPS];
-            const int ve = __builtin_amdgcn_readfirstlane(((const int*)tail)[32]);
-            const bool plain = __builtin_amdgcn_readfirstlane(((const int*)tail)[33]) != 0;
+            const bool plain = __builtin_amdgcn_readfirstlane(((const int*)tail)[kTailBad]) != 0;
+            // (values above 2^95 leave the sums no room for weights above 1)
+            const float grow = plain || __builtin_amdgcn_readfirstlane(((const int*)tail)[kTailMax]) < -80 ? 0.0f : 8.0f;
             float sv[16], tmax = NEG;
             if (!plain) {
                 f16v s0 = {}, s1 = {};
@@ -224,7 +240,7 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
                     s1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(k[s % PF][0], ql[s], s1, 0, 0, 0);
                 }
 #pragma unroll
-                for (uint32_t i = 0; i < 16; ++i) sv[i] = (s0[i] + s1[i]) * (qf * tail[8 * (i / 4) + 4 * h + i % 4]);
+                for (uint32_t i = 0; i < 16; ++i) sv[i] = (s0[i] + s1[i]) * (qf * tail[kTailK + 8 * (i / 4) + 4 * h + i % 4]);
             } else {
 #pragma unroll
                 for (uint32_t i = 0; i < 16; ++i) {
@@ -245,15 +261,13 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
             tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
             // a new reference only where the largest score has grown by 2^8
             // (the weights then stay below 2^8): the sums are seldom rescaled
-            if (__builtin_amdgcn_ballot_w64(tmax > m + 8.0f) || ve < eref) {
+            if (__builtin_amdgcn_ballot_w64(tmax > m + grow)) {
                 const float m_new = fmaxf(m, tmax), md_new = m_new == NEG ? 0.0f : m_new;
                 // (nothing seen yet: the sums are zeros)
                 const float alpha = m == NEG ? 0.0f : __builtin_amdgcn_exp2f(md - md_new);
                 l *= alpha;
-                const float f = ldexpf(alpha, min(ve - eref, 0));
 #pragma unroll
-                for (uint32_t b = 0; b < NB; ++b) acc[b] *= f;
-                eref = min(eref, ve);
+                for (uint32_t b = 0; b < NB; ++b) acc[b] *= alpha;
                 m = m_new;
                 md = md_new;
             }
@@ -264,15 +278,23 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
                 l += p[i];
             }
             if (!plain) {
-                const float pf = pf_pow2(6 + eref - ve);
-                const h8_t* vo = op + OPS / 2;  // (piece n: step n / NB of block n % NB)
+                const h8_t* vo = op + OPS / 2;
                 auto piece = [&](uint32_t n, h8_t (&v)[2]) {
-                    v[0] = vo[(n % NB * 2 + n / NB) * 128];
-                    v[1] = vo[(n % NB * 2 + n / NB) * 128 + 64];
+                    v[0] = vo[n * 128];
+                    v[1] = vo[n * 128 + 64];
                 };
                 h8_t v[PF][2], ph[2], pl[2];
 #pragma unroll
                 for (uint32_t n = 0; n < PF - 1; ++n) piece(n, v[n]);
+                float wmax = 0.0f;
+#pragma unroll
+                for (uint32_t i = 0; i < 16; ++i) {
+                    p[i] *= tail[kTailV + 8 * (i / 4) + 4 * h + i % 4];
+                    wmax = fmaxf(wmax, p[i]);
+                }
+                // (at least -111: below, f32 itself has no more bits)
+                const int ew = max(-111, __builtin_amdgcn_frexp_expf(fmaxf(wmax, __shfl_xor(wmax, 32, 64))));
+                const float pf = pf_pow2(15 - ew), of = pf_pow2(ew - 15);
 #pragma unroll
                 for (uint32_t s = 0; s < 2; ++s) {
                     float ps[8];
@@ -281,18 +303,24 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
                     pf_split(ps, pf, ph[s], pl[s]);
                 }
 #pragma unroll
-                for (uint32_t n = 0; n < 2 * NB; ++n) {
-                    const uint32_t b = n % NB, s = n / NB;
-                    if (n + PF - 1 < 2 * NB) piece(n + PF - 1, v[(n + PF - 1) % PF]);
-                    __builtin_amdgcn_sched_barrier(0);
-                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][1], ph[s], acc[b], 0, 0, 0);
-                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][0], pl[s], acc[b], 0, 0, 0);
-                    acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][0], ph[s], acc[b], 0, 0, 0);
+                for (uint32_t b = 0; b < NB; ++b) {
+                    f16v o = {};
+#pragma unroll
+                    for (uint32_t s = 0; s < 2; ++s) {
+                        const uint32_t n = 2 * b + s;
+                        if (n + PF - 1 < 2 * NB) piece(n + PF - 1, v[(n + PF - 1) % PF]);
+                        __builtin_amdgcn_sched_barrier(0);
+                        o = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][1], ph[s], o, 0, 0, 0);
+                        o = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][0], pl[s], o, 0, 0, 0);
+                        o = __builtin_amdgcn_mfma_f32_32x32x16_f16(v[n % PF][0], ph[s], o, 0, 0, 0);
+                    }
+#pragma unroll
+                    for (uint32_t i = 0; i < 16; ++i) acc[b][i] = fmaf(o[i], of, acc[b][i]);
                 }
             } else {
 #pragma unroll
                 for (uint32_t i = 0; i < 16; ++i) {
-                    const float mine = ldexpf(p[i], 6 + eref), other = __shfl_xor(mine, 32, 64);
+                    const float mine = p[i], other = __shfl_xor(mine, 32, 64);
 #pragma unroll
                     for (uint32_t o = 0; o < 2; ++o) {  // the positions of both halves
                         const uint32_t pos = p0 + 8 * (i / 4) + 4 * o + i % 4;
@@ -323,7 +351,7 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
         for (uint32_t g = 0; g < 4; ++g) {
             f32x4 v;
 #pragma unroll
-            for (uint32_t i = 0; i < 4; ++i) v[i] = ldexpf(acc[b][4 * g + i], -6 - eref);
+            for (uint32_t i = 0; i < 4; ++i) v[i] = acc[b][4 * g + i];
             *(f32x4*)(o + 32 * b + 8 * g + 4 * h) = a.nsp == 1 ? v / l : v;
         }
     if (a.nsp > 1 && h == 0) {

@@ -95,6 +95,52 @@ def test_prefill_attention_scales(ctx):
     assert np.all(np.abs(got - ref) <= 1e-5 * mag)
 
 
+def check_values(ctx, q, kc, vc, M, H, KVH, hd, S, q_start):
+    """Each output within 1e-5 of the values that its query weights, Σ p·|v|."""
+    args = (M, H, KVH, hd, S, S, q_start)
+    got = run(ctx, q.ravel(), kc.ravel(), vc.ravel(), 1, M, S, H, KVH, hd, S, q_start)[0]
+    ref = ora.causal_attention(q.ravel(), kc.ravel(), vc.ravel(), *args)
+    mag = ora.causal_attention(q.ravel(), kc.ravel(), np.abs(vc).ravel(), *args)
+    err = np.abs(got - ref)
+    assert np.all(err <= 1e-5 * mag), f"{(err / np.maximum(mag, 1e-300)).max():.1e}"
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("r", [10, 16, 24, 32, 60, -30])
+def test_prefill_attention_outweighed_values(ctx, hd, r):
+    """Values 2^r times the others' whose softmax weight is e^-20·2^-r: in a
+    record of their own at the start, and beside others at the end of one."""
+    rng = np.random.default_rng(20 + abs(r))
+    H, KVH, M, S = 2, 1, 40, 500
+    q, kc, vc = (rng.standard_normal((n, hd)).astype(np.float32) for n in (M * H, S, S))
+    q[:, 0], kc[:, 0] = np.sqrt(hd), 0
+    for at in (slice(0, 32), slice(440, 448)):
+        kc[at, 0] = -20 - max(r, 0) * np.log(2)
+        vc[at] *= np.float32(2.0 ** r)
+    check_values(ctx, q, kc, vc, M, H, KVH, hd, S, S - M)
+
+
+@pytest.mark.parametrize("std", [1.0, 1e-2, 1e-6, 1e-30])
+def test_prefill_attention_zero_values(ctx, std):
+    """Records and single positions of all-zero values (padding) among small ones."""
+    rng = np.random.default_rng(21)
+    hd, H, KVH, M, S = 64, 4, 2, 50, 410
+    q, kc, vc = (rng.standard_normal((n, hd)).astype(np.float32) for n in (M * H, KVH * S, KVH * S))
+    vc = (vc * std).astype(np.float32).reshape(KVH, S, hd)
+    vc[:, :32] = vc[:, 96:160] = vc[:, 330] = 0
+    check_values(ctx, q, kc, vc, M, H, KVH, hd, S, S - M)
+
+
+@pytest.mark.parametrize("r", [24, 40, 100])
+def test_prefill_attention_large_later_values(ctx, r):
+    """A value of 2^r leaves the queries before it, in its record too, as they are."""
+    rng = np.random.default_rng(22)
+    hd, H, KVH, M = 128, 2, 1, 70
+    q, kc, vc = (rng.standard_normal((n, hd)).astype(np.float32) for n in (M * H, M, M))
+    vc[31] *= np.float32(2.0 ** r)
+    check_values(ctx, q, kc, vc, M, H, KVH, hd, M, 0)
+
+
 def test_prefill_attention_infinities(ctx):
     """A key of -inf score leaves its position out, one of +inf makes the rows
     that see it NaN, an infinite value its element infinite: as in f32
