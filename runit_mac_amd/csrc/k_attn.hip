@@ -384,11 +384,10 @@ RT_DEV void attn_pf_merge(const AttnPfArgs& a) {
     f32x4 o = {0, 0, 0, 0};
 #pragma unroll
     for (uint32_t s = 0; s < RT_ATTN_MQ_NSP_MAX; ++s) {
-        const float f = s >= a.nsp || mj[s] == -__builtin_huge_valf() ? 0.0f : __builtin_amdgcn_exp2f(mj[s] - M);
-        if (f != 0.0f) {  // (an empty range, and one that the others outweigh, adds nothing)
-            L += f * lj[s];
-            o += f * oj[s];
-        }
+        // (an empty range adds zeros; one that the others outweigh its NaN, if it has one)
+        const float f = mj[s] == -__builtin_huge_valf() ? 0.0f : __builtin_amdgcn_exp2f(mj[s] - M);
+        L += s < a.nsp ? f * lj[s] : 0.0f;
+        o += s < a.nsp ? f * oj[s] : f32x4{0, 0, 0, 0};
     }
     const uint32_t row = c / G, head = blockIdx.y * G + c % G;
     *(f32x4*)(a.out + ((size_t)(blockIdx.z * a.q_len + row) * a.H + head) * HD + d) = o / L;

@@ -165,6 +165,31 @@ def test_prefill_attention_infinities(ctx):
     assert np.all(np.isnan(got[70:]))
 
 
+@pytest.mark.parametrize("what", ["range", "outweighed key", "outweighed value"])
+def test_prefill_attention_nan_ranges(ctx, what):
+    """A NaN reaches every query that sees it, whatever the weight of the range
+    of positions that holds it (520 positions: ranges of 128): a range of NaN
+    keys, a NaN key and an infinite value (0·inf) beside keys of scores below
+    all others by 300."""
+    rng = np.random.default_rng(23)
+    hd, H, KVH, M, S = 64, 2, 1, 40, 520
+    q, kc, vc = (rng.standard_normal((n, hd)).astype(np.float32) for n in (M * H, S, S))
+    q[:, 0], kc[:, 0] = np.sqrt(hd), 0
+    kc[128:256, 0] = -300
+    ref = ora.causal_attention(q.ravel(), kc.ravel(), vc.ravel(), M, H, KVH, hd, S, S, S - M).reshape(M * H, hd)
+    element = np.ones(hd, bool)
+    if what == "range":
+        kc[128:256] = np.nan
+    elif what == "outweighed key":
+        kc[130] = np.nan
+    else:
+        vc[130, 9] = np.inf
+        element = np.arange(hd) == 9
+    got = run(ctx, q.ravel(), kc.ravel(), vc.ravel(), 1, M, S, H, KVH, hd, S, S - M)[0].reshape(M * H, hd)
+    assert np.all(np.isnan(got[:, element]))
+    assert np.all(np.abs(got - ref)[:, ~element] <= 1e-5 * np.abs(vc[:, ~element]).max(initial=0))
+
+
 def test_prefill_attention_capture():
     """Captured in a context whose workspace is not sized the call keeps the
     kernel that needs none; after an eager call it is captured in this form,
