@@ -324,7 +324,7 @@ RT_DEV void attn_pf(const AttnPfArgs& a) {
 #pragma unroll
                     for (uint32_t o = 0; o < 2; ++o) {  // the positions of both halves
                         const uint32_t pos = p0 + 8 * (i / 4) + 4 * o + i % 4;
-                        if (pos >= a.kv) continue;
+                        if (pos >= lim) continue;  // (0·inf is none of its column's)
                         const float pp = o == h ? mine : other;
                         const float* vp = a.vc + ((size_t)seq * a.stride + pos) * HD + 4 * h;
 #pragma unroll

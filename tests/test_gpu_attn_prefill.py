@@ -159,7 +159,7 @@ def test_prefill_attention_infinities(ctx):
     for lo, hi, keys in ((0, 20, clean[1]), (20, 70, low)):
         ref = ora.causal_attention(clean[0], keys.ravel(), clean[2].ravel(), M, H, KVH, hd, M, S, 0).reshape(M, H, hd)
         for r in range(lo, hi):
-            e = np.arange(hd) != 9 if r >= 32 else np.ones(hd, bool)  # (0·inf in the record of value 45 is NaN)
+            e = np.arange(hd) != 9 if r >= 45 else np.ones(hd, bool)  # (the rows before 45 share its record)
             assert np.max(np.abs(got[r][:, e] - ref[r][:, e])) <= 1e-5 * np.abs(clean[2]).max(), r
     assert np.all(np.isinf(got[45:70, :, 9]))
     assert np.all(np.isnan(got[70:]))
