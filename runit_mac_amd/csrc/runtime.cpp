@@ -317,8 +317,9 @@ struct rt_ctx {
     uint32_t gemm_splits = 0;    // RUNIT_GEMM_SPLITS=n: the f16 GEMM's K splits forced (A/B)
     bool attn_w = true;          // RUNIT_ATTN_W=0: the token's RoPE attention on attn_split (A/B)
     bool attn_mq = true;         // RUNIT_ATTN_MQ=0: multi-query attention on attn_split per row (A/B)
-    // RUNIT_ATTN_PF_WORK: query heads × positions from which a prompt's attention takes the f16
-    // form (0: every one it can; tests, A/B); RUNIT_ATTN_PF_NSP: its ranges (0: planned)
+    // RUNIT_ATTN_PF_WORK: query heads × positions from which a prompt's attention may take the f16
+    // form (attn_pf_launch's rule; 0: every one it can; tests, A/B); RUNIT_ATTN_PF_NSP: its ranges
+    // (0: planned)
     uint64_t attn_pf_work = 3000000;
     uint32_t attn_pf_nsp = 0;
     uint32_t attn_mq_nsp = 0, attn_mq_w = 0;  // probe: forced ranges / waves (0: planned)
@@ -3800,6 +3801,12 @@ int rt_argmax_rows_first_f32(rt_ctx* c, const float* in, uint32_t* result, uint3
 }
 
 
+// Key ranges of k_attn_mq for `pairs` column groups over `tiles` of 16 positions.
+static uint32_t attn_mq_ranges(uint64_t pairs, uint32_t tiles) {
+    if (pairs >= 256) return 1;
+    return std::max<uint32_t>(1, std::min<uint32_t>({(uint32_t)(256 / pairs), tiles / 4, RT_ATTN_MQ_NSP_MAX}));
+}
+
 // The multi-query attention on the matrix cores (k_attn_mq_f32_hd*): plan and
 // launch; kLsDecline where the per-row kernel is the better one.  in_part:
 // the split partials in the context's second scratch buffer (c->part) instead
@@ -3830,10 +3837,7 @@ static int attn_mq_launch(rt_ctx* c, AttnArgs a, uint32_t batch, uint32_t q_len,
         const uint64_t pairs = cols * num_kv_heads * batch;
         const uint32_t tiles = (std::min<uint32_t>(kv_len, q_start + q_len) + 15) / 16;
         const uint32_t wmax = rt_attn_mq_wmax(head_dim);
-        uint32_t nsp = 1;
-        if (pairs < 256)
-            nsp = std::max<uint32_t>(1, std::min<uint32_t>({(uint32_t)(256 / pairs), tiles / 4,
-                                                            RT_ATTN_MQ_NSP_MAX}));
+        uint32_t nsp = attn_mq_ranges(pairs, tiles);
         if (c->attn_mq_nsp) nsp = std::min({c->attn_mq_nsp, tiles, RT_ATTN_MQ_NSP_MAX});
         const uint32_t chunk = (tiles + nsp - 1) / nsp;
         nsp = (tiles + chunk - 1) / chunk;
@@ -3890,15 +3894,10 @@ static int attn_pf_launch(rt_ctx* c, const AttnArgs& a, uint32_t batch, uint32_t
     if (!c->attn_mq || (head_dim != 64 && head_dim != 128) || batch > 65535) return kLsDecline;
     const uint32_t kv = std::min<uint64_t>(a.kv_len, (uint64_t)a.q_start + a.q_len);
     const uint64_t rows = (uint64_t)batch * a.q_len * a.H, cols = (uint64_t)a.q_len * (a.H / a.KVH);
-    // From 1,024 positions on: fewer are too little work for its three launches
-    // (28 heads of 128, 128 queries: 20 against 11 µs; 256: 28 / 27), and the
-    // f16 pairs' own error, which does not grow with the positions, exceeds the
-    // f32 form's there (300 queries: 1.6e-7 against 1.3e-7; after 500
-    // positions level at 2.2e-7; after 1,000 2.5e-7 against 2.8e-7; 512 after
-    // 1,536 3.4e-7 against 4.3e-7).  And from 3e6 scores on: 64 queries after
-    // 1,000 (1.9e6) 29 against 28 µs, 128 after 1,000 (4.0e6) 33 / 38, 64 after
-    // 4,000 (7.3e6) 53 / 67, 512 after 1,536 (29e6) 79 / 182, 2,048 alone 155 /
-    // 482; 14 heads of 64, 300 after 1,000 (5.5e6) 27 / 40.
+    // From 1,024 positions on: the f16 pairs' own error, which does not grow with
+    // the positions, exceeds the f32 form's below (28 heads of 128, 300 queries:
+    // 1.65e-7 against 1.56e-7; 128 after 1,000 2.5e-7 against 2.9e-7; 512 after
+    // 1,536 2.6e-7 against 4.2e-7).
     if (c->attn_pf_work && (kv < 1024 || rows * kv < c->attn_pf_work)) return kLsDecline;
     // ranges of the positions for about two workgroups on every CU, each of at
     // least 4 records of 32; twice as many where the first query sees less than
@@ -3910,6 +3909,30 @@ static int attn_pf_launch(rt_ctx* c, const AttnArgs& a, uint32_t batch, uint32_t
     const uint64_t slots = (a.q_start < kv / 2 ? 4ull : 2ull) * c->cu_count;
     uint32_t nsp = std::max<uint64_t>(1, std::min<uint64_t>({slots / wgs, tiles / 4, RT_ATTN_MQ_NSP_MAX}));
     if (c->attn_pf_nsp) nsp = std::min({c->attn_pf_nsp, tiles, RT_ATTN_MQ_NSP_MAX});
+    if (c->attn_pf_work) {
+        // Where the estimated time is 5% below k_attn_mq's: few columns of a KV
+        // head fill neither its workgroups nor, with 8 ranges at most, the CUs,
+        // while every position is prepared all the same.  Fitted to 1,000 random
+        // calls of 1-1,500 queries, batches to 16, caches to 20,000 positions: of
+        // 681 that it takes 10 are slower than there, by 12% at most, of the others
+        // 32 would be faster, by 18%.  µs here against there: 28 heads of 128 512
+        // queries after 1,536 81 / 189, 2,048 alone 148 / 473, 64 after 4,000 57 /
+        // 69; 14 heads of 64 300 after 1,000 28 / 42; left there: 28 heads of 128
+        // 16 after 8,192 85 / 44, 64 sequences of one after 4,095 633 / 187.
+        const double cu = c->cu_count, items = (double)wgs * nsp;
+        const double last = kv - (a.q_len - 1) / 2.0, seen = std::max(last, kv / 2.0) / kv;
+        const double rec = (head_dim + 59) / 128.0 * tiles / nsp;  // of a workgroup
+        const double run = items <= cu       ? 3.4 + 1.4 * rec
+                           : items <= 2 * cu ? 3.4 + 2.1 * rec
+                                             : items / (2 * cu) * (3.4 + 2.1 * rec * seen);
+        const double pf = 14.5 + run + 3.0e-6 * batch * a.KVH * kv * head_dim +
+                          (nsp > 1 ? 2.2e-6 * rows * head_dim * nsp : 0.0);
+        const uint64_t pairs = (cols + 15) / 16 * a.KVH * batch;
+        const uint32_t t16 = (kv + 15) / 16, r16 = attn_mq_ranges(pairs, t16);
+        const uint64_t per = (pairs * r16 + c->cu_count - 1) / c->cu_count;  // workgroups of a CU
+        const double mq = 16.0 + 0.41 / 128 * head_dim * per * ((t16 + r16 - 1) / r16) * (0.68 * seen + 0.32);
+        if (pf > 0.95 * mq) return kLsDecline;
+    }
     if (wgs * nsp > 0x7FFFFF00ull) return kLsDecline;
     const size_t o_bytes = (size_t)batch * a.KVH * tiles * (head_dim * 16 + 64) * 16;
     const size_t parts = nsp > 1 ? (size_t)wgs * nsp * 128 : 0;

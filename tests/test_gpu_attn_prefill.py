@@ -222,3 +222,39 @@ def test_prefill_attention_capture():
                 call()  # (eager; sizes the workspace the first time)
                 ctx.flush()
             del g
+
+
+@pytest.mark.parametrize("hd,H,KVH,batch,M,start,form", [
+    (128, 28, 4, 1, 512, 1536, "pf"),
+    (64, 14, 2, 1, 300, 1000, "pf"),
+    (128, 28, 4, 4, 32, 2000, "pf"),
+    (128, 28, 4, 1, 300, 500, "mq"),    # fewer than 1,024 positions
+    (64, 14, 2, 1, 64, 4000, "mq"),     # few columns of a KV head
+    (128, 28, 4, 1, 16, 8192, "mq"),
+    (64, 8, 8, 16, 8, 4000, "mq"),
+    (128, 28, 4, 8, 4, 4092, "mq"),
+])
+def test_prefill_attention_rule(hd, H, KVH, batch, M, start, form):
+    """Which calls of a context without switches take this form: not those of
+    few queries a sequence, whose caches its preparation would rewrite for
+    little (k_attn_mq is up to four times as fast there)."""
+    S = start + M
+    with d.HipContext() as ctx:
+        bufs = [ctx.buffer_from(np.ones(n, np.float32)) for n in (batch * M * H * hd, batch * KVH * S * hd)]
+        bo = ctx.new_buffer(4 * batch * M * H * hd)
+        d.flash_attention_f32(ctx, bufs[0], bufs[1], bufs[1], bo, batch, M, S, H, KVH, hd, S, start)
+        ctx.flush()
+        assert d.last_launch_name(ctx).startswith(f"k_attn_{form}_")
+        assert np.max(np.abs(bo.read(np.float32, batch * M * H * hd) - 1)) <= 1e-5
+
+
+def test_prefill_attention_rules_own_range():
+    """A prompt chunk that takes this form without switches, against the oracle."""
+    rng = np.random.default_rng(24)
+    hd, H, KVH, M, S, start = 64, 14, 2, 300, 1300, 1000
+    q = rng.standard_normal(M * H * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal(KVH * S * hd).astype(np.float32) for _ in range(2))
+    with d.HipContext() as c:
+        got = run(c, q, kc, vc, 1, M, S, H, KVH, hd, S, start)[0]
+    ref = ora.causal_attention(q, kc, vc, M, H, KVH, hd, S, S, start)
+    assert np.max(np.abs(got - ref)) <= 1e-5 * np.abs(vc).max()
