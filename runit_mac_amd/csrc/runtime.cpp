@@ -2059,32 +2059,57 @@ static bool gemmw_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_ro
     return true;
 }
 
-// Whether a call whose K the staged forms do not tile takes the wide form
-// (the other way: a GEMV a row, for Q8_0 the unstaged GEMM).  Its time hardly
-// depends on the rows below 64; the GEMVs' is theirs times the rows: Q4_0
+// Whether a call whose K the staged forms do not tile takes the wide form.
+// The other formats' alternative is a GEMV a row, whose time is theirs times
+// the rows, where the wide form's hardly depends on them below 64: Q4_0
 // 5000×2080 at 3 / 5 / 32 rows 20 / 34 / 211 against 21 / 20 / 21 µs, 18944×
 // 3616 45 / 73 / 456 against 44 / 41 / 43; Q6_K 3584×18688 at 3 / 4 / 32 57 /
-// 77 / 598 against 52 / 52 / 53, 896×1280 17 / 22 / 177 against 18.  The
-// unstaged GEMM, Q8_0 at 8 / 32 rows: 18944×3616 62 / 80 against 56 / 57 µs,
-// 5000×2080 25 / 31 against 23 / 24, but 896×1056 12 / 14 against 16 / 17.
-static bool gemm_wide_untiled(const rt_ctx* c, const GemmFmt& f, uint32_t m_rows, uint32_t n, uint32_t k) {
-    if (m_rows > c->gemm_wide_min) return true;
-    if (f.blk_bytes == 34) return m_rows > 4 && (uint64_t)n * k >= 1u << 23;
-    return m_rows > (f.blk_bytes == 210 ? 3 : 4);
+// 77 / 598 against 52 / 52 / 53, 896×1280 17 / 22 / 177 against 18.
+// Q8_0's is the unstaged GEMM, which gains from a few short rounds of its
+// workgroups (16 weight rows × 32 activation rows) and from rows of an odd
+// number of blocks, whose loads the wide form cannot align (17 sizes of K from
+// 32 to 18,912, 15 of N, 19 of M; µs there against here):
+//   above 32 rows, one round: 64×896×544 13 / 15, ×1056 16 / 16, ×1568 18 / 18,
+//   ×2080 20 / 19, even ×1088 16 / 14; several: 64×2560×544 19 / 16, 128×1280×
+//   1056 24 / 19; K of few blocks: 128×3584×288 20 / 22, at 12 rounds 25 / 24;
+//   16-32 rows: 18944×544 24 / 28, 12000×1568 29 / 26, 5000×1056 24 / 19;
+//   5-16 rows, odd: 3584×4832 23 / 30, 12000×1568 28 / 31, 18944×2080 42 / 38;
+//   even: 2048×4160 22 / 20, 18944×576 23 / 20.
+// A set of several matrices (alone: false) is one preparation, one launch and
+// one sum in the wide form, three launches a matrix in the other: Q/K/V of 33
+// rows and K = 544 38 / 16 µs, gate and up 30 / 17, gate and up of 1,056 at 5
+// rows 30 / 30, of 2,080 54 / 34.
+static bool gemm_wide_untiled(const rt_ctx* c, const GemmFmt& f, uint32_t m_rows, uint32_t n, uint32_t k,
+                              bool alone) {
+    if (f.blk_bytes != 34) return m_rows > (f.blk_bytes == 210 ? 3 : 4);
+    const uint32_t blocks = k / 32;
+    const uint64_t weights = (uint64_t)n * k;
+    const bool odd = blocks % 2;
+    if (m_rows <= 4) return false;
+    if (!c->gemm_wide_work) return true;  // (every call it can: tests, A/B)
+    if (m_rows <= c->gemm_wide_min) {
+        if (!alone || !odd) return weights >= 1u << 23;
+        return m_rows <= 16 ? weights >= 1u << 25 : weights >= 1u << 23 && blocks >= 25;
+    }
+    if (!alone) return true;
+    const uint64_t rounds = ((uint64_t)(n + 15) / 16 * ((m_rows + 31) / 32) + c->cu_count - 1) / c->cu_count;
+    if (blocks < 17) return rounds > 9;
+    return rounds > 1 || !odd || blocks >= (n < 256 ? 17u : 50u);
 }
 
 // Plans the f16 form: 8 activation rows per group (MG ∈ {1, 2, 4}), hi/lo
 // f16 operands prepared by k_gemm_xh_prep*_mg*.  Returns kLsDecline where
 // the staged layout does not apply (the caller then takes the other forms).
-// work: rows × weights of the whole call (0: of this matrix; UINT64_MAX: the
-// wide form, for a call of which one matrix has no other).  The wide form takes
+// work: rows × weights of the whole call (0: this matrix is all of it;
+// UINT64_MAX: the wide form, for a call of which one matrix has no other).  The wide form takes
 // calls above gemm_wide_min rows of gemm_wide_work on, and those whose K the
 // stages here do not tile.
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                       uint32_t k, Gemm3Plan& p, uint64_t work = 0) {
     p = Gemm3Plan{};
     const uint32_t cu = (uint32_t)c->cu_count;
-    if (!work) work = (uint64_t)m_rows * n * k;
+    const bool alone = work == 0;
+    if (alone) work = (uint64_t)m_rows * n * k;
     if ((work == UINT64_MAX || (m_rows > c->gemm_wide_min && work >= c->gemm_wide_work)) &&
         gemmw_plan(c, f, w, m_rows, n, k, p))
         return RT_OK;
@@ -2108,7 +2133,7 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     }
     const uint32_t seg = NB * f.blk_bytes, vb = seg % 16 == 0 ? 16 : (seg % 8 == 0 ? 8 : 4);
     if (nblk % NB != 0 || !aligned(w, 16) || row_bytes % vb != 0 || c->gemm_direct)
-        return gemm_wide_untiled(c, f, m_rows, n, k) && gemmw_plan(c, f, w, m_rows, n, k, p) &&
+        return gemm_wide_untiled(c, f, m_rows, n, k, alone) && gemmw_plan(c, f, w, m_rows, n, k, p) &&
                        ws_holds(c, p.a_bytes + p.e_bytes + p.s_bytes + p.p_bytes)
                    ? RT_OK
                    : kLsDecline;
@@ -2793,7 +2818,7 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
                   (!rope || (1024 % rope->head_dim == 0 && rope->head_dim % 4 == 0 && rope->head_dim <= 512 && n[0] % 4 == 0 && n[1] % 4 == 0 &&
                              c->gemm_rope));
     uint64_t work = 0;
-    for (uint32_t i = 0; i < count; ++i) work += (uint64_t)m_rows * n[i] * k;
+    for (uint32_t i = 0; count > 1 && i < count; ++i) work += (uint64_t)m_rows * n[i] * k;
     for (uint32_t i = 0; shared && i < count; ++i) shared = !bias || aligned(bias[i], 8);
     for (uint32_t i = 0; shared && i < count; ++i) {
         int st = gemm3_plan(c, *f[i], w[i], m_rows, n[i], k, pl[i], work);
@@ -3004,8 +3029,12 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         return s;
     };
     int st = plan((uint64_t)m_rows * h * (qd + 3ull * ff));
-    if (st == RT_OK && (po.MG == 8 || pg.MG == 8 || pu.MG == 8 || pd.MG == 8))
+    if (st == RT_OK && (po.MG == 8 || pg.MG == 8 || pu.MG == 8 || pd.MG == 8)) {
         st = plan(UINT64_MAX);  // (one of them may only have the wide form)
+        // 4 rows (only a Q6_K matrix takes it there) and K of up to 4 blocks: the sets
+        // (Q4_K_M, 2,304 and 6,912 wide, 4 rows: 66 / 69 µs; Q8_0 of 32 and 128, 64 rows 32 / 35)
+        if (m_rows <= 4 || h < 160) return plan_only ? RT_OK : sets();
+    }
     if (st == kLsDecline ||
         (st == RT_OK && (pg.MG != po.MG || pu.MG != po.MG || pd.MG != po.MG ||
                          (po.MG == 8 ? fg != fu : pg.splits != pu.splits))))

@@ -93,6 +93,28 @@ def test_wide_set_few_rows_of_mixed_formats(ctx, m):
         check_close(y.read(np.float32, m * n), ref.ravel(), sabs.ravel(), f"{f} of a mixed set of {m} rows")
 
 
+@pytest.mark.parametrize("m,n,k,wide", [
+    (33, 896, 544, False), (128, 896, 1056, False), (64, 2048, 1568, False), (100, 3584, 288, False),
+    (8, 3584, 3616, False), (16, 12000, 1568, False), (20, 18944, 544, False), (4, 18944, 2080, False),
+    (33, 896, 1088, True), (33, 896, 2080, True), (64, 2560, 544, True), (256, 896, 1056, True),
+    (20, 12000, 1056, True), (8, 18944, 2080, True), (8, 8200, 1088, True),
+])
+def test_q8_0_untiled_k_form(m, n, k, wide):
+    """Which Q8_0 GEMMs of a K that the stages do not tile take the wide form in
+    a context without switches: not those that the unstaged kernel's few
+    workgroups finish sooner."""
+    with d.HipContext() as c:
+        w, raw = device_weights(c, "q8_0", n, k, 1020 + m)
+        x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+        y = c.new_buffer(4 * m * n)
+        d.gemm_q8_0_f32(c, w, c.buffer_from(x), y, m, n, k)
+        assert d.last_launch_name(c).startswith("k_gemm_q8_0_") != wide, d.last_launch_name(c)
+        c.flush()
+        rows = [0, m // 2, m - 1]
+        ref, sabs = ora.gemv("q8_0", raw, x[rows], n, k)
+        check_close(y.read(np.float32, m * n).reshape(m, n)[rows].ravel(), ref.ravel(), sabs.ravel(), f"{m}x{n}x{k}")
+
+
 @pytest.mark.parametrize("fmt", ["q8_0", "q4kg"])
 def test_wide_gemm_whole_and_split_tiles(ctx, fmt):
     """520 tiles: 512 of one workgroup each and 8 with K split (256 compute
