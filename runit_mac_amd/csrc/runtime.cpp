@@ -2097,22 +2097,31 @@ static bool gemm_wide_untiled(const rt_ctx* c, const GemmFmt& f, uint32_t m_rows
     return rounds > 1 || !odd || blocks >= (n < 256 ? 17u : 50u);
 }
 
+// gemm3_plan's work for a call of which one matrix has only the wide form, and
+// for one whose workspace does not hold that form.
+constexpr uint64_t kWideWork = UINT64_MAX, kStagedWork = UINT64_MAX - 1;
+
 // Plans the f16 form: 8 activation rows per group (MG ∈ {1, 2, 4}), hi/lo
 // f16 operands prepared by k_gemm_xh_prep*_mg*.  Returns kLsDecline where
 // the staged layout does not apply (the caller then takes the other forms).
 // work: rows × weights of the whole call (0: this matrix is all of it;
-// UINT64_MAX: the wide form, for a call of which one matrix has no other).  The wide form takes
-// calls above gemm_wide_min rows of gemm_wide_work on, and those whose K the
-// stages here do not tile.
+// kWideWork, kStagedWork).  The wide form takes calls above gemm_wide_min rows
+// of gemm_wide_work on, and those whose K the stages here do not tile, while
+// the workspace holds it.
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                       uint32_t k, Gemm3Plan& p, uint64_t work = 0) {
     p = Gemm3Plan{};
     const uint32_t cu = (uint32_t)c->cu_count;
     const bool alone = work == 0;
     if (alone) work = (uint64_t)m_rows * n * k;
-    if ((work == UINT64_MAX || (m_rows > c->gemm_wide_min && work >= c->gemm_wide_work)) &&
-        gemmw_plan(c, f, w, m_rows, n, k, p))
-        return RT_OK;
+    auto wide = [&] {
+        return work != kStagedWork && gemmw_plan(c, f, w, m_rows, n, k, p) &&
+               ws_holds(c, p.a_bytes + p.e_bytes + p.s_bytes + p.p_bytes);
+    };
+    if (work == kWideWork || (m_rows > c->gemm_wide_min && work >= c->gemm_wide_work)) {
+        if (wide()) return RT_OK;
+        p = Gemm3Plan{};
+    }
     const uint32_t groups = (m_rows + 7) / 8;
     const uint32_t MG = std::min<uint32_t>(f.max_mg_f16, groups <= 1 ? 1 : groups <= 2 ? 2 : 4);
     const uint32_t nchunks = (m_rows + 8 * MG - 1) / (8 * MG);
@@ -2133,10 +2142,7 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
     }
     const uint32_t seg = NB * f.blk_bytes, vb = seg % 16 == 0 ? 16 : (seg % 8 == 0 ? 8 : 4);
     if (nblk % NB != 0 || !aligned(w, 16) || row_bytes % vb != 0 || c->gemm_direct)
-        return gemm_wide_untiled(c, f, m_rows, n, k, alone) && gemmw_plan(c, f, w, m_rows, n, k, p) &&
-                       ws_holds(c, p.a_bytes + p.e_bytes + p.s_bytes + p.p_bytes)
-                   ? RT_OK
-                   : kLsDecline;
+        return gemm_wide_untiled(c, f, m_rows, n, k, alone) && wide() ? RT_OK : kLsDecline;
     // Q6_K: 128-row tiles with one operand and one weight buffer
     const bool q6 = f.blk_bytes == 210;
     const bool w8ok = !q6 || (c->gemm_q6w8 >> (MG == 4 ? 0 : MG == 2 ? 1 : 2) & 1);
@@ -2820,21 +2826,28 @@ static int gemm_set_impl(rt_ctx* c, uint32_t count, const char* const* fmts, con
     uint64_t work = 0;
     for (uint32_t i = 0; count > 1 && i < count; ++i) work += (uint64_t)m_rows * n[i] * k;
     for (uint32_t i = 0; shared && i < count; ++i) shared = !bias || aligned(bias[i], 8);
-    for (uint32_t i = 0; shared && i < count; ++i) {
-        int st = gemm3_plan(c, *f[i], w[i], m_rows, n[i], k, pl[i], work);
-        if (st == RT_OK && i && pl[i].MG != pl[0].MG && (pl[i].MG == 8 || pl[0].MG == 8) && work != UINT64_MAX) {
-            work = UINT64_MAX;  // one of them only has the wide form
-            i = UINT32_MAX;
-            continue;
+    // (RT_OK: every matrix planned on one form; *mixed: one on the wide form, one not)
+    auto plan = [&](uint64_t wk, bool* mixed) {
+        for (uint32_t i = 0; i < count; ++i) {
+            const int st = gemm3_plan(c, *f[i], w[i], m_rows, n[i], k, pl[i], wk);
+            if (st != RT_OK) return st;
+            if (pl[i].MG == pl[0].MG) continue;
+            *mixed = pl[i].MG == 8 || pl[0].MG == 8;
+            return (int)kLsDecline;
         }
+        return (int)RT_OK;
+    };
+    if (shared) {
+        bool mixed = false;
+        int st = plan(work, &mixed);
+        if (mixed) st = plan(kWideWork, &mixed);  // one of them only has the wide form
+        if (st == RT_OK && pl[0].MG == 8) {
+            st = gemm_set_wide(c, count, f, pl, w, y, n, bias, res, x, m_rows, k, gamma, eps, xn, silu_pair, rope);
+            if (st != kLsDecline) return st;
+        }
+        if (st == kLsDecline) st = plan(kStagedWork, &mixed);
         if (st != RT_OK && st != kLsDecline) return st;
-        shared = st == RT_OK && pl[i].MG == pl[0].MG;
-    }
-    if (shared && pl[0].MG == 8) {
-        const int st = gemm_set_wide(c, count, f, pl, w, y, n, bias, res, x, m_rows, k, gamma, eps, xn,
-                                     silu_pair, rope);
-        if (st != kLsDecline) return st;
-        shared = false;
+        shared = st == RT_OK;
     }
     if (!shared) {
         // the separate launches: norm, one GEMM per matrix, then the
@@ -2974,13 +2987,14 @@ int rt_gemm_qkv_rope_f32(rt_ctx* c, const char* fmt_q, const void* w_q, const ch
 // rt_gemm_ffn_block_f32.  plan_only: report in *shared whether the shared
 // form applies, launching nothing; pa: the O projection's input given as
 // multi-query attention partials (merged in its operand preparation) instead
-// of att (shared form only).
+// of att (shared form only).  staged: not the wide form, whose workspace is
+// not there.
 static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const char* fmt_gate,
                           const void* w_gate, const char* fmt_up, const void* w_up,
                           const char* fmt_down, const void* w_down, const float* att, float* x,
                           float* x_mid, const float* gamma, float eps, float* g, float* u,
                           float* xn, uint32_t m_rows, uint32_t h, uint32_t qd, uint32_t ff,
-                          bool plan_only, bool* shared, const PrepAttnHost* pa) {
+                          bool plan_only, bool* shared, const PrepAttnHost* pa, bool staged = false) {
     if (shared) *shared = false;
     if (!c) return fail(nullptr, RT_ERR_DISPATCH, "kernel dispatch error: null context");
     if (m_rows == 0) return RT_OK;
@@ -3028,12 +3042,17 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         if (s == RT_OK) s = gemm3_plan(c, *fd, w_down, m_rows, h, ff, pd, work);
         return s;
     };
-    int st = plan((uint64_t)m_rows * h * (qd + 3ull * ff));
+    auto on_stages = [&] {
+        return ffn_block_impl(c, fmt_o, w_o, fmt_gate, w_gate, fmt_up, w_up, fmt_down, w_down, att, x, x_mid, gamma,
+                              eps, g, u, xn, m_rows, h, qd, ff, plan_only, shared, pa, true);
+    };
+    int st = plan(staged ? kStagedWork : (uint64_t)m_rows * h * (qd + 3ull * ff));
     if (st == RT_OK && (po.MG == 8 || pg.MG == 8 || pu.MG == 8 || pd.MG == 8)) {
-        st = plan(UINT64_MAX);  // (one of them may only have the wide form)
+        st = plan(kWideWork);  // (one of them may only have the wide form)
         // 4 rows (only a Q6_K matrix takes it there) and K of up to 4 blocks: the sets
         // (Q4_K_M, 2,304 and 6,912 wide, 4 rows: 66 / 69 µs; Q8_0 of 32 and 128, 64 rows 32 / 35)
         if (m_rows <= 4 || h < 160) return plan_only ? RT_OK : sets();
+        if (po.MG != 8 || pg.MG != 8 || pu.MG != 8 || pd.MG != 8) return on_stages();
     }
     if (st == kLsDecline ||
         (st == RT_OK && (pg.MG != po.MG || pu.MG != po.MG || pd.MG != po.MG ||
@@ -3067,7 +3086,7 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
     }
     const size_t off_pd = total;
     total += parts(pd, h);
-    if (MG == 8 && !ws_holds(c, total)) return plan_only ? RT_OK : sets();
+    if (MG == 8 && !ws_holds(c, total)) return on_stages();
     if (plan_only) {
         if (shared) *shared = true;
         return RT_OK;

@@ -215,3 +215,74 @@ def test_wide_gemm_few_rows_capture():
                     call()
                     ctx.flush()
                 del g
+
+
+def _sized_context(nbytes, former):
+    """A context whose workspace holds about nbytes; former: without the wide form."""
+    if former:
+        os.environ["RUNIT_GEMM_WIDE_WORK"] = str(1 << 62)
+    try:
+        c = d.HipContext()
+    finally:
+        os.environ.pop("RUNIT_GEMM_WIDE_WORK", None)
+    nrec = nbytes // 4224 | 1  # (the unstaged Q8_0 GEMM takes 4,224 bytes of it a record of 32 rows)
+    w, x, y = c.new_buffer(34 * nrec), c.new_buffer(4 * 32 * 32 * nrec), c.new_buffer(4 * 32)
+    d.gemm_q8_0_f32(c, w, x, y, 32, 1, 32 * nrec)
+    c.flush()
+    return c
+
+
+@pytest.mark.parametrize("what", ["gemm", "set", "pair", "block"])
+def test_wide_gemm_capture_in_a_workspace_of_the_staged_form(what):
+    """A call that takes the wide form is captured wherever the staged forms
+    alone could be, in workspaces from too small for these to enough for both,
+    and every replay gives the result."""
+    m, h, ff = (70, 1024, 8192) if what == "block" else (70, 2048, 11520)
+    rng = np.random.default_rng(15)
+    x = rng.standard_normal((m, h if what == "block" else ff)).astype(np.float32)
+    accepted = []
+    for mb in (2, 4, 5, 6, 7, 8, 10, 12, 16, 24, 40):
+        ok = []
+        for former in (True, False):
+            with _sized_context(mb << 20, former) as c:
+                xb = c.buffer_from(x)
+                if what == "block":
+                    W = [device_weights(c, "q4k", n, k, 1030 + i)[0] for i, (n, k) in enumerate(((h, h), (ff, h), (ff, h), (h, ff)))]
+                    at, xm, xn, g, u = (c.new_buffer(4 * m * n) for n in (h, h, h, ff, ff))
+                    at.write(0.1 * x)
+                    gam = c.buffer_from(np.ones(h, np.float32))
+                    out = xb
+                    call = lambda: d.gemm_ffn_block_f32(c, ["q4k"] * 4, *W, at, xb, xm, gam, 1e-6, g, u, xn, m, h, h, ff)
+                    size = m * h
+                else:
+                    W = [device_weights(c, "q4k", h, ff, 1040 + i)[0] for i in range(2)]
+                    ys = [c.new_buffer(4 * m * h) for _ in range(2)]
+                    out, size = ys[0], m * h
+                    if what == "gemm":
+                        call = lambda: d.gemm_q4k_f32(c, W[0], xb, ys[0], m, h, ff)
+                    else:
+                        call = lambda: d.gemm_set_f32(c, ["q4k"] * 2, W, ys, [h, h], xb, m, ff, silu_pair=what == "pair")
+                c.capture_begin()
+                try:
+                    call()
+                    ok.append(True)
+                except d.KernelError:
+                    ok.append(False)
+                graph = c.capture_end()
+                if not ok[-1]:
+                    continue
+                got = []
+                for i in range(3):  # two replays, then eager
+                    if what == "block":
+                        xb.write(x)
+                    else:
+                        out.write(np.zeros(size, np.float32))
+                    graph.launch() if i < 2 else call()
+                    c.flush()
+                    got.append(out.read(np.float32, size))
+                tol = 1e-5 * np.abs(got[2]).max()  # (the eager call may take the other form)
+                assert np.max(np.abs(got[0] - got[2])) <= tol and np.max(np.abs(got[1] - got[2])) <= tol
+                del graph
+        assert ok[1] or not ok[0], f"{mb} MB: refused"
+        accepted.append(ok[1])
+    assert accepted[-1] and not accepted[0]
