@@ -286,3 +286,165 @@ def test_wide_gemm_capture_in_a_workspace_of_the_staged_form(what):
         assert ok[1] or not ok[0], f"{mb} MB: refused"
         accepted.append(ok[1])
     assert accepted[-1] and not accepted[0]
+
+
+@pytest.fixture(scope="module")
+def staged():
+    """A context without the wide form for K that the staged forms tile."""
+    os.environ["RUNIT_GEMM_WIDE_WORK"] = str(1 << 62)
+    try:
+        c = d.HipContext()
+    finally:
+        del os.environ["RUNIT_GEMM_WIDE_WORK"]
+    yield c
+    c.close()
+
+
+def _block64(fmts, raws, att, x, gamma, eps, h, qd, ff):
+    """The layer after its attention in f64 (projection inputs rounded to f32):
+    x_mid and x with the Σ|w·x| of the O and down sums."""
+    y, so = ora.gemv(fmts[0], raws[0], att, h, qd)
+    xm = x + y
+    xn = xm / np.sqrt((xm * xm).mean(1, keepdims=True) + eps) * gamma
+    g, _ = ora.gemv(fmts[1], raws[1], xn, ff, h)
+    u, _ = ora.gemv(fmts[2], raws[2], xn, ff, h)
+    y, sd = ora.gemv(fmts[3], raws[3], g / (1 + np.exp(-g)) * u, h, ff)
+    return xm, so, xm + y, sd
+
+
+def _check_block(ctx, staged, fmts, m, h, qd, ff, call, att, rows, seed):
+    """call(context, weights, x, x_mid, gamma, eps, g, u, xn) on both contexts:
+    x_mid within 1e-6 of its sums (as the GEMMs above) and its own rounding, x
+    within 1e-5 of the down sums (the product silu(gate)·up carries the error of
+    its own two sums, some ten times smaller than they), and other bits than the
+    staged forms': the wide ones ran."""
+    x0 = np.random.default_rng(seed).standard_normal((m, h)).astype(np.float32)
+    gamma = np.linspace(0.5, 1.5, h, dtype=np.float32)
+    outs = []
+    for c in (ctx, staged):
+        W = [device_weights(c, f, n, k, seed + i)
+             for i, (f, n, k) in enumerate(zip(fmts, (h, ff, ff, h), (qd, h, h, ff)))]
+        x, xm = c.buffer_from(x0), c.new_buffer(4 * m * h)
+        g, u, xn = c.new_buffer(4 * m * ff), c.new_buffer(4 * m * ff), c.new_buffer(4 * m * h)
+        call(c, [w for w, _ in W], x, xm, c.buffer_from(gamma), 1e-6, g, u, xn)
+        c.flush()
+        outs.append((xm.read(np.float32, m * h).reshape(m, h), x.read(np.float32, m * h).reshape(m, h)))
+    xm, so, x, sd = _block64(fmts, [r for _, r in W], att[rows], x0[rows], gamma, 1e-6, h, qd, ff)
+    for got, ref, s, tol, what in ((outs[0][0], xm, so, 1e-6, "x_mid"), (outs[0][1], x, sd, 1e-5, "x")):
+        err = np.abs(got[rows] - ref)
+        bound = tol * s + 2.0 ** -23 * np.abs(ref)
+        assert np.all(err <= bound), f"{what}: {(err / bound).max():.2f} of the bound"
+        assert np.all(np.isfinite(got)), what
+    if h % 128 == 0:  # (the staged forms tile it)
+        assert not np.array_equal(outs[0][0], outs[1][0]) and not np.array_equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("fmts,m,h,qd,ff", [
+    (("q4k", "q4k", "q4k", "q6k"), 33, 1024, 1024, 2048),
+    (("q8_0", "q8_0", "q8_0", "q8_0"), 65, 1056, 1120, 2592),  # (K that nothing else tiles, on both)
+    (("q8_0", "q8_0", "q8_0", "q8_0"), 65, 896, 4608, 2560),   # preparations of up to and over 4,096
+    (("q4kg", "q4kg", "q4kg", "q6kg"), 130, 4352, 512, 5120),
+    (("q4k", "q4k", "q4k", "q4k"), 440, 20480, 512, 512),      # O: 560 tiles, 512 of them whole
+])
+def test_wide_block(ctx, staged, fmts, m, h, qd, ff):
+    att = np.random.default_rng(m).standard_normal((m, qd)).astype(np.float32)
+
+    def call(c, W, x, xm, gamma, eps, g, u, xn):
+        d.gemm_ffn_block_f32(c, fmts, *W, c.buffer_from(att), x, xm, gamma, eps, g, u, xn, m, h, qd, ff)
+
+    _check_block(ctx, staged, fmts, m, h, qd, ff, call, att, [0, m // 2, m - 1], 1050 + m)
+
+
+@pytest.mark.parametrize("fmts,hd,heads,kvh,m,start", [
+    (("q4k", "q4k", "q4k", "q6k"), 128, 8, 2, 33, 300),
+    (("q8_0", "q8_0", "q8_0", "q8_0"), 64, 14, 2, 70, 200),
+    (("q4kg", "q4kg", "q4kg", "q6kg"), 128, 36, 4, 34, 200),   # O's K of 4,608
+])
+def test_wide_block_with_folded_attention(ctx, staged, fmts, hd, heads, kvh, m, start):
+    """The attention's key-range partials merged in the wide form's preparation."""
+    h, qd, ff, S = 768, heads * hd, 1536, start + m
+    rng = np.random.default_rng(m)
+    q = rng.standard_normal((m, qd)).astype(np.float32)
+    kc, vc = (rng.standard_normal((kvh, S, hd)).astype(np.float32) for _ in range(2))
+    att = ora.causal_attention(q, kc, vc, m, heads, kvh, hd, S, S, start).reshape(m, qd)
+
+    def call(c, W, x, xm, gamma, eps, g, u, xn):
+        at = c.buffer_from(np.full(m * qd, 7.0, np.float32))
+        d.gemm_attn_ffn_block_f32(c, c.buffer_from(q), c.buffer_from(kc), c.buffer_from(vc), S, heads, kvh, hd, S,
+                                  start, at, fmts, *W, x, xm, gamma, eps, g, u, xn, m, h, ff)
+        c.flush()
+        assert np.all(at.read(np.float32, m * qd) == 7.0)  # (the folded form does not write it)
+
+    _check_block(ctx, staged, fmts, m, h, qd, ff, call, att, [0, m // 2, m - 1], 1060 + m)
+
+
+@pytest.mark.parametrize("what", ["bias", "rope", "pair", "residual"])
+def test_wide_set_whole_and_split_tiles(ctx, staged, what):
+    """Sets of 520 tiles and more, 512 of one workgroup each, the others with K
+    split: the sums of the split ones alone are added, in 16-byte units (rows of
+    a multiple of 4), against the oracle and with other bits than the staged
+    form's."""
+    m, k, hd = 35, 512, 64
+    ns = {"bias": [256 * 400, 256 * 100 + 4, 256 * 19 + 8], "rope": [256 * 400, 256 * 100 + 64, 256 * 19 + 64],
+          "pair": [128 * 519 + 4] * 2, "residual": [256 * 519 + 4]}[what]
+    if what == "rope":
+        ns[2] = ns[1]
+    rng = np.random.default_rng(16)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    biases = [(0.1 * rng.standard_normal(n)).astype(np.float16) for n in ns]
+    rows, outs = [0, m - 1], []
+    for c in (ctx, staged):
+        W = [device_weights(c, "q8_0", n, k, 1070 + i) for i, n in enumerate(ns)]
+        xb, ys = c.buffer_from(x), [c.new_buffer(4 * m * n) for n in ns]
+        bb = [c.buffer_from(b.view(np.uint16)) for b in biases]
+        if what == "rope":
+            kvh = ns[1] // hd
+            xn, kc, vc = c.new_buffer(4 * m * k), *(c.new_buffer(4 * kvh * m * hd) for _ in range(2))
+            gam = c.buffer_from(np.ones(k, np.float32))
+            d.gemm_qkv_rope_f32(c, ["q8_0"] * 3, *[w for w, _ in W], *bb, xb, gam, 0.0, xn, *ys, kc, vc, m, k, *ns[:2],
+                                hd, 0, 10000.0, m)
+            c.flush()
+            x = xn.read(np.float32, m * k).reshape(m, k)
+            got = [ys[0].read(np.float32, m * ns[0]).reshape(m, -1)] + [
+                b.read(np.float32, kvh * m * hd).reshape(kvh, m, hd).transpose(1, 0, 2).reshape(m, -1) for b in (kc, vc)]
+        else:
+            kw = {"bias": dict(biases=bb), "pair": dict(silu_pair=True),
+                  "residual": dict(res=c.buffer_from(np.tile(biases[0].astype(np.float32), (m, 1))))}[what]
+            d.gemm_set_f32(c, ["q8_0"] * len(ns), [w for w, _ in W], ys, ns, xb, m, k, **kw)
+            c.flush()
+            got = [y.read(np.float32, m * n).reshape(m, n) for y, n in zip(ys, ns)][:1 if what == "pair" else 3]
+        outs.append(got)
+    refs = [ora.gemv("q8_0", raw, x[rows], n, k) for (_, raw), n in zip(W, ns)]
+    if what == "pair":
+        ffn_check(outs[0][0][rows].ravel(), refs[0][0].ravel(), refs[0][1].ravel(), refs[1][0].ravel(),
+                  refs[1][1].ravel(), what)
+    else:
+        for i, (g, (ref, sabs), b) in enumerate(zip(outs[0], refs, biases)):
+            ref = ref + b.astype(np.float64)
+            if what == "rope" and i < 2:  # pairs (j, j + 32) of each head, row r at position r
+                a = np.array(rows)[:, None, None] / 10000.0 ** (2 * np.arange(32) / hd)
+                t = ref.reshape(2, -1, 2, 32)
+                ref = np.stack([t[:, :, 0] * np.cos(a) - t[:, :, 1] * np.sin(a),
+                                t[:, :, 0] * np.sin(a) + t[:, :, 1] * np.cos(a)], 2).reshape(2, -1)
+                sabs = np.repeat(sabs.reshape(2, -1, 2, 32).sum(2, keepdims=True), 2, 2).reshape(2, -1)
+                sabs += np.abs(ref).max()  # (angles of up to 34 radians in f32: 4e-6 of the pair)
+            check_close(g[rows].ravel(), ref.ravel(), sabs.ravel(), f"{what} {i}", extra=1e-6 * np.abs(ref).ravel())
+    assert any(not np.array_equal(a, b) for a, b in zip(*outs))
+
+
+@pytest.mark.parametrize("fmt,m,n,k,wide", [("q8_0", 124, 3584, 3584, False), ("q8_0", 125, 3584, 3584, True),
+                                            ("q4k", 32, 18944, 3584, False), ("q4k", 33, 18944, 3584, True)])
+def test_wide_gemm_rule(ctx, staged, fmt, m, n, k, wide):
+    """From 33 rows and 1.6e9 rows x weights on a context without switches takes
+    the wide form: its result is that form's, bit for bit."""
+    x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    outs = []
+    with d.HipContext() as plain:
+        for c in (plain, ctx, staged):
+            w, _ = device_weights(c, fmt, n, k, 1080)
+            y = c.new_buffer(4 * m * n)
+            getattr(d, f"gemm_{fmt}_f32")(c, w, c.buffer_from(x), y, m, n, k)
+            c.flush()
+            outs.append(y.read(np.float32, m * n))
+    assert np.array_equal(outs[0], outs[1 if wide else 2])
+    assert m <= 32 or not np.array_equal(outs[1], outs[2])
