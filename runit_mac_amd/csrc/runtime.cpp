@@ -279,8 +279,8 @@ struct rt_ctx {
     size_t max_lds = 65536;
     std::string err = "no error";
     bool capturing = false;
-    // RUNIT_GEMM_WIDE_WORK: rows × weights from which a call takes the wide form (A/B).  Below,
-    // its tiles leave the grid to K splits: Q8_0 64×3584×3584 (0.8e9) 24.2 against 22.6 µs,
+    // RUNIT_GEMM_WIDE_WORK: rows × weights from which a call takes the wide form (A/B; 0: every one it
+    // can).  Below, its tiles leave the grid to K splits: Q8_0 64×3584×3584 (0.8e9) 24.2 against 22.6 µs,
     // 300×4864×1024 (1.5e9) 30 / 25, 128×3584×3584 (1.6e9) 28.5 / 32.7, 33×18944×3584 (2.2e9) 40 / 57
     uint64_t gemm_wide_work = 1600000000ull;
     uint32_t gemm_wide_min = 32;  // RUNIT_GEMM_WIDE_MIN: rows above which a GEMM takes the wide form (A/B)
