@@ -2097,6 +2097,29 @@ static bool gemm_wide_untiled(const rt_ctx* c, const GemmFmt& f, uint32_t m_rows
     return rounds > 1 || !odd || blocks >= (n < 256 ? 17u : 50u);
 }
 
+// From how many times gemm_wide_work on a single matrix that the staged forms
+// tile too takes the wide form.  Blocks of 32 elements gain less there (their
+// scale is applied a record, the super-blocks' 128 elements), and a short K
+// leaves it little between a workgroup's start and end, 4 and 5 bits least of
+// all (m×n×k, staged / wide form): Q8_0 192×8192×1024 (1.6e9) 23.8 / 28.6 µs,
+// 448×4864×1024 (2.2e9) 9% ahead; ggml Q4_0 160×12000×1024 (2.0e9) 28% behind,
+// 256×8192×1536 (3.2e9) 31.6 / 37.6, 128×13928×2048 (3.7e9) 5% behind, 256×
+// 13928×2048 (7.3e9) 14% ahead; from K = 2,560 on ahead or level from 1.6e9 on.
+static double gemm_wide_alone_factor(const GemmFmt& f, uint32_t k) {
+    const double kk = k;
+    if (f.blk_el != 32) return 1.0;
+    if (f.blk_bytes == 34) return k < 1152 ? std::max(1.0, kk / 800) : 1.0;
+    if (!strcmp(f.name, "q4_0")) return k < 2048 ? std::max(1.0, kk / 760) : 1.0;
+    return k < 2560 ? std::max(1.0, kk / 500) : 1.0;
+}
+// ... and a layer block of such matrices: Q8_0 96×(1536, 4096) (2.0e9) 6%
+// behind, 112 rows level; Q4_0 160×(896, 4864) (2.2e9) 9% behind, 192 rows 5%
+// ahead; ggml Q4_0 and Q5_0 224×(1024, 4096) (3.1e9) 9% behind, 320 rows 3%
+// ahead.  (Q4_K 33×(2048, 8192), 1.8e9: 81 / 66 µs.)
+static double gemm_wide_block_factor(const GemmFmt& f) {
+    return f.blk_el != 32 ? 1.0 : f.blk_bytes == 34 || !strcmp(f.name, "q4_0") ? 1.5 : 2.25;
+}
+
 // gemm3_plan's work for a call of which one matrix has only the wide form, and
 // for one whose workspace does not hold that form.
 constexpr uint64_t kWideWork = UINT64_MAX, kStagedWork = UINT64_MAX - 1;
@@ -2106,7 +2129,7 @@ constexpr uint64_t kWideWork = UINT64_MAX, kStagedWork = UINT64_MAX - 1;
 // the staged layout does not apply (the caller then takes the other forms).
 // work: rows × weights of the whole call (0: this matrix is all of it;
 // kWideWork, kStagedWork).  The wide form takes calls above gemm_wide_min rows
-// of gemm_wide_work on, and those whose K the stages here do not tile, while
+// of gemm_wide_work (times the factors above) on, and those whose K the stages here do not tile, while
 // the workspace holds it.
 static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_rows, uint32_t n,
                       uint32_t k, Gemm3Plan& p, uint64_t work = 0) {
@@ -2118,8 +2141,16 @@ static int gemm3_plan(rt_ctx* c, const GemmFmt& f, const void* w, uint32_t m_row
         return work != kStagedWork && gemmw_plan(c, f, w, m_rows, n, k, p) &&
                ws_holds(c, p.a_bytes + p.e_bytes + p.s_bytes + p.p_bytes);
     };
-    if (work == kWideWork || (m_rows > c->gemm_wide_min && work >= c->gemm_wide_work)) {
-        if (wide()) return RT_OK;
+    if (work == kWideWork || (m_rows > c->gemm_wide_min &&
+                              work >= c->gemm_wide_work * (alone ? gemm_wide_alone_factor(f, k) : 1.0))) {
+        // Not two 64-row chunks for 65-96 rows over tiles that fill half of the
+        // CUs and are too short to split: the staged form runs three of 32
+        // (18944×1024 / 2048 at 96 rows: Q8_0 25 / 40 against 31 / 54 µs, ggml
+        // Q4_0 23 / 37 against 33 / 54, Q4_K 25 / 41 against 29 / 48; 112 rows of
+        // Q8_0 23% the other way)
+        if (wide() && !(alone && c->gemm_wide_work && m_rows > 64 && m_rows <= 96 && k < 3072 && p.splits == 1 &&
+                        p.base > cu / 2 && p.base <= cu))
+            return RT_OK;
         p = Gemm3Plan{};
     }
     const uint32_t groups = (m_rows + 7) / 8;
@@ -3046,7 +3077,9 @@ static int ffn_block_impl(rt_ctx* c, const char* fmt_o, const void* w_o, const c
         return ffn_block_impl(c, fmt_o, w_o, fmt_gate, w_gate, fmt_up, w_up, fmt_down, w_down, att, x, x_mid, gamma,
                               eps, g, u, xn, m_rows, h, qd, ff, plan_only, shared, pa, true);
     };
-    int st = plan(staged ? kStagedWork : (uint64_t)m_rows * h * (qd + 3ull * ff));
+    double factor = 1.0;
+    for (const GemmFmt* f : {fo, fg, fu, fd}) factor = std::max(factor, gemm_wide_block_factor(*f));
+    int st = plan(staged ? kStagedWork : (uint64_t)(m_rows * (double)h * (qd + 3.0 * ff) / factor));
     if (st == RT_OK && (po.MG == 8 || pg.MG == 8 || pu.MG == 8 || pd.MG == 8)) {
         st = plan(kWideWork);  // (one of them may only have the wide form)
         // 4 rows (only a Q6_K matrix takes it there) and K of up to 4 blocks: the sets

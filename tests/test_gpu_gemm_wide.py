@@ -432,11 +432,19 @@ def test_wide_set_whole_and_split_tiles(ctx, staged, what):
     assert any(not np.array_equal(a, b) for a, b in zip(*outs))
 
 
-@pytest.mark.parametrize("fmt,m,n,k,wide", [("q8_0", 124, 3584, 3584, False), ("q8_0", 125, 3584, 3584, True),
-                                            ("q4k", 32, 18944, 3584, False), ("q4k", 33, 18944, 3584, True)])
+@pytest.mark.parametrize("fmt,m,n,k,wide", [
+    ("q8_0", 124, 3584, 3584, False), ("q8_0", 125, 3584, 3584, True),
+    ("q4k", 32, 18944, 3584, False), ("q4k", 33, 18944, 3584, True),
+    ("q8_0", 192, 8192, 1024, False), ("q8_0", 256, 8192, 1024, True),       # short K of 32-element blocks
+    ("q4_0", 160, 12000, 1024, False), ("q4_0", 192, 12000, 1024, True),
+    ("q4_0g", 128, 13928, 2048, False), ("q4_0g", 256, 13928, 2048, True), ("q5_0", 65, 10000, 2560, True),
+    ("q4k", 96, 18944, 2048, False), ("q4k", 97, 18944, 2048, True), ("q8_0", 65, 18944, 1536, False),
+])
 def test_wide_gemm_rule(ctx, staged, fmt, m, n, k, wide):
-    """From 33 rows and 1.6e9 rows x weights on a context without switches takes
-    the wide form: its result is that form's, bit for bit."""
+    """Which GEMMs of a K that the staged forms tile take the wide form in a
+    context without switches: from 33 rows and 1.6e9 rows x weights on, more
+    where the staged form stays ahead longer.  The result is that form's, bit
+    for bit."""
     x = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
     outs = []
     with d.HipContext() as plain:
@@ -448,3 +456,23 @@ def test_wide_gemm_rule(ctx, staged, fmt, m, n, k, wide):
             outs.append(y.read(np.float32, m * n))
     assert np.array_equal(outs[0], outs[1 if wide else 2])
     assert m <= 32 or not np.array_equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("fmt,m,h,ff,wide", [("q8_0", 96, 1536, 4096, False), ("q8_0", 192, 1536, 4096, True),
+                                             ("q4_0g", 224, 1024, 4096, False), ("q4_0g", 320, 1024, 4096, True),
+                                             ("q4k", 33, 2048, 8192, True)])
+def test_wide_block_rule(ctx, staged, fmt, m, h, ff, wide):
+    """The same of layer blocks."""
+    rng = np.random.default_rng(m)
+    x, att = (rng.standard_normal((m, h)).astype(np.float32) for _ in range(2))
+    outs = []
+    with d.HipContext() as plain:
+        for c in (plain, ctx, staged):
+            W = [device_weights(c, fmt, n, k, 1090 + i)[0] for i, (n, k) in enumerate(((h, h), (ff, h), (ff, h), (h, ff)))]
+            xb, xm, xn, g, u = c.buffer_from(x), *(c.new_buffer(4 * m * n) for n in (h, h, ff, ff))
+            d.gemm_ffn_block_f32(c, [fmt] * 4, *W, c.buffer_from(att), xb, xm, c.buffer_from(np.ones(h, np.float32)),
+                                 1e-6, g, u, xn, m, h, h, ff)
+            c.flush()
+            outs.append(xb.read(np.float32, m * h))
+    assert np.array_equal(outs[0], outs[1 if wide else 2])
+    assert not np.array_equal(outs[1], outs[2])
