@@ -476,3 +476,30 @@ def test_wide_block_rule(ctx, staged, fmt, m, h, ff, wide):
             outs.append(xb.read(np.float32, m * h))
     assert np.array_equal(outs[0], outs[1 if wide else 2])
     assert not np.array_equal(outs[1], outs[2])
+
+
+@pytest.mark.parametrize("fmts,m,h,ff,sets", [(("q4k", "q4k", "q4k", "q6k"), 4, 768, 2304, True),
+                                              (("q4k", "q4k", "q4k", "q6k"), 5, 768, 2304, False),
+                                              (("q8_0",) * 4, 64, 96, 288, True), (("q8_0",) * 4, 64, 160, 480, False)])
+def test_wide_block_of_untiled_k_or_its_sets(fmts, m, h, ff, sets):
+    """4 rows, and hidden sizes below 160, run as the three sets, in their launches."""
+    x = np.random.default_rng(m).standard_normal((m, h)).astype(np.float32)
+    counts, outs = [], []
+    with d.HipContext() as c:
+        W = [device_weights(c, f, n, k, 1100 + i)[0] for i, (f, n, k) in enumerate(zip(fmts, (h, ff, ff, h), (h, h, h, ff)))]
+        gam = c.buffer_from(np.ones(h, np.float32))
+        for block in (True, False):
+            at, xb, xm, xn, g, u = (c.buffer_from(np.ones((m, n), np.float32)) for n in (h, h, h, h, ff, ff))
+            xb.write(x)
+            n0 = d.launch_count(c)
+            if block:
+                d.gemm_ffn_block_f32(c, fmts, *W, at, xb, xm, gam, 1e-6, g, u, xn, m, h, h, ff)
+            else:
+                d.gemm_set_f32(c, fmts[:1], W[:1], [xm], [h], at, m, h, res=xb)
+                d.gemm_set_f32(c, fmts[1:3], W[1:3], [g, u], [ff, ff], xm, m, h, gamma=gam, eps=1e-6, xn=xn, silu_pair=True)
+                d.gemm_set_f32(c, fmts[3:], W[3:], [xb], [h], g, m, ff, res=xm)
+            counts.append(d.launch_count(c) - n0)
+            c.flush()
+            outs.append(xb.read(np.float32, m * h))
+    assert (counts[0] == counts[1]) == sets, counts
+    assert np.max(np.abs(outs[0] - outs[1])) <= 1e-5 * np.abs(outs[1]).max()
